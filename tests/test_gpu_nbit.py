@@ -45,13 +45,39 @@ def test_single_type(dev, ty, D):
         _check(got, exp)
 
 
+@pytest.mark.parametrize("ty", TYPES + [orc.FP8])
+@pytest.mark.parametrize("dims", [[20, 12, 24, 40, 48, 60, 72, 96, 100, 112, 120],
+                                  [5, 4, 136, 144, 200, 248, 252], [264, 392, 500, 512],
+                                  [516, 680, 1000, 1024]])
+def test_ragged_widths(dev, ty, dims):
+    """Widths that the group's lanes do not divide, on each instance of the
+    launch (lanes per bag follow the widest table), with output columns at odd
+    elements; the last table's last row ends the buffer."""
+    if ty in (orc.INT4, orc.INT2):
+        dims = [d + d % 2 if ty == orc.INT4 else -(-d // 4) * 4 for d in dims]
+    print(f"[case] nbit ragged ty={ty} dims={dims}", flush=True)
+    rng = np.random.default_rng(ty * 31 + dims[-1])
+    T, rows = len(dims), [23] * len(dims)
+    inp = random_tbe(rng, T, 37, dims, rows, 25)
+    tys = [ty] * T
+    buf, w_off = build_weights(rng, tys, dims, rows)
+    iw = rng.uniform(0, 1, size=inp.N).astype(np.float32)
+    W = torch.from_numpy(buf).to(dev)
+    for weights, out_f16 in ((None, True), (iw, True), (None, False)):
+        exp = orc.nbit_forward(buf, w_off, tys, inp.D_offsets, inp.B, inp.indices, inp.offsets,
+                               0, indice_weights=weights, out_f16=out_f16)
+        got = nbit_forward_gpu(dev, W, w_off, tys, dims, inp.indices, inp.offsets, 0,
+                               out_f16=out_f16, indice_weights=weights)
+        _check(got, exp)
+
+
 @pytest.mark.parametrize("ebits,ebias", [(4, 7), (5, 15), (3, 3)])
 @pytest.mark.parametrize("D", [8, 16, 24, 32, 96, 128, 256, 520])
 def test_fp8_tables(dev, ebits, ebias, D):
     """FP8 (hfp8) tables: every code decodes exactly and the rows add in index
     order, as in the oracle (bit-exact to FBGEMM's FP8 CPU kernel), so SUM and
-    MEAN, weighted or not, fp16 or fp32 out, match bit for bit; D = 24 and
-    520 take the general path."""
+    MEAN, weighted or not, fp16 or fp32 out, match bit for bit; D = 24, 96
+    and 520 take the ragged-width path."""
     print(f"[case] nbit fp8 ebits={ebits} bias={ebias} D={D}", flush=True)
     rng = np.random.default_rng(ebits * 1000 + D)
     inp = random_tbe(rng, 2, 19, [D, D], [37, 5], 25)
