@@ -55,6 +55,34 @@ def test_fused_nbit_round_trip_bits(dev, bits, D):
     np.testing.assert_array_equal(qh.cpu().numpy(), orc.quantize_fused_nbit(xh.float().numpy(), bits))
 
 
+@pytest.mark.parametrize("bits", [2, 4, 8, "fused8"])
+@pytest.mark.parametrize("rows,D", [(3, 33), (37, 62), (5, 65), (130, 129), (7, 255), (6, 257),
+                                    (5, 511), (3, 514), (9, 1021), (2, 1026), (3, 2050), (2, 4099)])
+def test_row_codec_lane_edges(dev, bits, rows, D):
+    """Widths around the lane and word counts at which the row kernels change
+    (words per lane, lanes per row, the wide kernel), partial last words, and
+    row counts that leave groups idle; encode and decode bit-exact."""
+    print(f"[case] row codec bits={bits} rows={rows} D={D}", flush=True)
+    x = _rows(np.random.default_rng(D), rows, D)
+    ops = torch.ops.fbgemm
+    for src in (torch.from_numpy(x), torch.from_numpy(x).half()):
+        ref = src.float().numpy()
+        if bits == "fused8":
+            q = ops.FloatOrHalfToFused8BitRowwiseQuantized(src.to(dev))
+            exp = orc.quantize_fused8bit(ref)
+            d, h = ops.Fused8BitRowwiseQuantizedToFloat(q), ops.Fused8BitRowwiseQuantizedToHalf(q)
+            back = orc.dequantize_fused8bit(exp)
+        else:
+            q = ops.FloatOrHalfToFusedNBitRowwiseQuantizedSBHalf(src.to(dev), bits)
+            exp = orc.quantize_fused_nbit(ref, bits)
+            d = ops.FusedNBitRowwiseQuantizedSBHalfToFloat(q, bits)
+            h = ops.FusedNBitRowwiseQuantizedSBHalfToHalf(q, bits)
+            back = orc.dequantize_fused_nbit(exp, bits, d.shape[1])
+        np.testing.assert_array_equal(q.cpu().numpy(), exp)
+        np.testing.assert_array_equal(d.cpu().numpy(), back)
+        np.testing.assert_array_equal(h.cpu().numpy(), back.astype(np.float16))
+
+
 @pytest.mark.parametrize("ebits,ebias", [(4, 7), (5, 15), (3, 3), (2, 1), (7, 0), (1, 0)])
 def test_hfp8_codecs(dev, ebits, ebias):
     """fbgemm::HFP8QuantizedToFloat on all 256 codes and FloatToHFP8Quantized on

@@ -93,6 +93,14 @@ __device__ __forceinline__ int64_t readlane_i64(int64_t v, int lane) {
 
 __device__ __forceinline__ int lane_id() { return __lane_id(); }
 
+// v, rounded to fp32: the compiler may fuse the operation that made v with a
+// conversion to fp16 into one instruction that rounds once, which differs from
+// the two roundings of the CPU kernels on a tie.
+__device__ __forceinline__ float fp32_value(float v) {
+  asm("" : "+v"(v));
+  return v;
+}
+
 // Sum over all 64 lanes (tree order fixed: deterministic).
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
