@@ -81,6 +81,26 @@ def test_bounds_check_large_batch_and_long_bags(dev, dtype, T, B, maxlen, long_b
     assert int(warn.item()) == exp_n
 
 
+@pytest.mark.parametrize("dtype", [torch.int64, torch.int32])
+@pytest.mark.parametrize("T,B", [(1, 1), (1, 257), (2, 2048), (1, 4096), (1, 4097), (3, 1366),
+                                 (40, 100), (2, 150000)])
+def test_bounds_check_tile_and_table_edges(dev, dtype, T, B):
+    """Bag counts around the single-tile limit (4096), blocks inside one table
+    (vector loads whose last vector is partial) and across several, and a batch
+    whose blocks take the most bags."""
+    print(f"[case] bounds_check edges {dtype} T={T} B={B}", flush=True)
+    rng = np.random.default_rng(T + B)
+    rows = rng.integers(50, 500, T)
+    idx, off = _case(rng, T, B, rows, 0.05, True)
+    exp_idx, exp_off, exp_n = orc.bounds_check_indices(rows, idx, off, 1)
+    gi, go = torch.from_numpy(idx).to(dev, dtype), torch.from_numpy(off).to(dev, dtype)
+    warn = torch.zeros(1, dtype=torch.int64, device=dev)
+    torch.ops.fbgemm.bounds_check_indices(torch.from_numpy(rows).to(dev), gi, go, 1, warn)
+    np.testing.assert_array_equal(gi.cpu().numpy(), exp_idx)
+    np.testing.assert_array_equal(go.cpu().numpy(), exp_off)
+    assert int(warn.item()) == exp_n
+
+
 def test_fatal_raises_and_repairs_nothing(dev):
     print("[case] bounds_check FATAL", flush=True)
     rng = np.random.default_rng(3)

@@ -12,14 +12,17 @@
 //   * each repaired entry (offset or index) adds one to warning[0];
 //   * FATAL repairs nothing and only counts (the host raises on a non-zero
 //     count); NONE does nothing.
-// Work: two launches, no zeroed state.  A tile kernel takes, one wave per
-// tile, the maximum of the clamped offsets of every tile of `tile` bags.  Then
-// a block owns `bpb` consecutive bags (32 to 256, by the mean bag length): it
-// rebuilds o' for them exactly (the maximum over earlier tiles and over the
-// earlier part of its own tile, then a block-wide max-scan), repairs its own
-// offsets, and checks the indices of its bags -- one contiguous range of
-// positions -- finding each position's bag by a binary search over the
-// repaired offsets in LDS.  Only the owner writes an offset; a neighbour that
+// Work: one launch, or two from kOneTile bags on, and no zeroed state.  A tile
+// kernel takes, one wave per tile, the maximum of the clamped offsets of every
+// tile of `tile` bags (a smaller batch is one tile, which needs none).  Then a
+// block owns `bpb` consecutive bags (32 to 256, so that the grid fills the
+// chip): it rebuilds o' for them exactly (the maximum over earlier tiles and
+// over the earlier part of its own tile, then a block-wide max-scan), repairs
+// its own offsets, and checks the indices of its bags -- one contiguous range
+// of positions.  A block whose bags are of one table compares them all with
+// that table's rows, 16 bytes of indices per load; at a table boundary each
+// position finds its bag by a binary search over the repaired offsets in LDS.
+// (10.5M int64 indices of 524k bags: 54 us with a search per position, 26 us.)  Only the owner writes an offset; a neighbour that
 // reads it before or after the repair computes the same o' (the maximum of a
 // prefix is unchanged when some of its entries are replaced by their own
 // prefix maxima), so no block waits on another.
@@ -40,6 +43,10 @@ namespace {
 
 constexpr int kMaxBagsPerBlock = 256;
 constexpr int kIdxPerThread = 4;  // index loads in flight per thread
+// Batches of at most this many bags are one tile: a block reads the offsets
+// before its own itself (16 loads per thread at most, from the L2) and the
+// tile launch is left out (its ~5 us are most of a small batch's check).
+constexpr int64_t kOneTile = 4096;
 
 template <typename I>
 __device__ __forceinline__ uint32_t clamp_off(I v, int64_t N) {
@@ -82,6 +89,7 @@ __global__ void __launch_bounds__(256)
   __shared__ uint32_t s_wmax[4];
   __shared__ uint32_t s_rep[kMaxBagsPerBlock + 1];
   __shared__ int64_t s_lim[kMaxBagsPerBlock];
+  __shared__ int64_t s_t[2];  // table of the block's first and last bag
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int64_t b0 = static_cast<int64_t>(blockIdx.x) * bpb;
   const int64_t b1 = b0 + bpb < nbags ? b0 + bpb : nbags;
@@ -92,6 +100,7 @@ __global__ void __launch_bounds__(256)
   const int64_t tb = b0 / tile;
   uint32_t carry = 0;
   for (int64_t t = tid; t < tb; t += 256) carry = umax(carry, tilemax[t]);
+#pragma unroll 4
   for (int64_t j = tb * tile + tid; j < b0; j += 256) carry = umax(carry, clamp_off(offsets[j], N));
   carry = wave_max(carry);
   if (lane == 0) s_red[w] = carry;
@@ -115,6 +124,8 @@ __global__ void __launch_bounds__(256)
       t = bag / B;
     }
     s_lim[tid] = rows[t];
+    if (tid == 0) s_t[0] = t;
+    if (tid == nb - 1) s_t[1] = t;
   }
   const uint32_t v = wave_incl_scan<MaxOp>(mine ? clamp_off(orig, N) : 0u);
   if (lane == 63) s_wmax[w] = v;
@@ -146,29 +157,60 @@ __global__ void __launch_bounds__(256)
   __syncthreads();
   // Indices of the block's bags: positions [o'[b0], o'[b1]).
   const int64_t p0 = s_rep[0], p1 = s_rep[nb];
-  for (int64_t base = p0; base < p1; base += 256 * kIdxPerThread) {
-    I idx[kIdxPerThread];
+  if (s_t[0] == s_t[1]) {  // block-uniform: one table
+    constexpr int V = 16 / sizeof(I);
+    typedef I IV __attribute__((ext_vector_type(V), aligned(sizeof(I))));
+    const int64_t lim = s_lim[0];
+    for (int64_t base = p0; base < p1; base += 256 * kIdxPerThread * V) {
+      IV x[kIdxPerThread];
 #pragma unroll
-    for (int k = 0; k < kIdxPerThread; ++k) {
-      const int64_t l = base + k * 256 + tid;
-      idx[k] = l < p1 ? indices[l] : I(0);
-    }
+      for (int k = 0; k < kIdxPerThread; ++k) {
+        const int64_t l = base + (k * 256 + tid) * V;
+        if (l + V <= p1) {
+          x[k] = *reinterpret_cast<const IV*>(indices + l);
+        } else {
 #pragma unroll
-    for (int k = 0; k < kIdxPerThread; ++k) {
-      const int64_t l = base + k * 256 + tid;
-      if (l >= p1) break;
-      int lo = 0, hi = nb;  // s_rep[lo] <= l < s_rep[hi]
-      while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (static_cast<int64_t>(s_rep[mid]) <= l)
-          lo = mid;
-        else
-          hi = mid;
+          for (int v = 0; v < V; ++v) x[k][v] = l + v < p1 ? indices[l + v] : I(0);
+        }
       }
-      const int64_t x = static_cast<int64_t>(idx[k]);
-      if (x < 0 || x >= s_lim[lo]) {
-        ++nbad;
-        if (fix) indices[l] = static_cast<I>(0);
+#pragma unroll
+      for (int k = 0; k < kIdxPerThread; ++k) {
+        const int64_t l = base + (k * 256 + tid) * V;
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+          const int64_t i = static_cast<int64_t>(x[k][v]);
+          if (l + v < p1 && (i < 0 || i >= lim)) {
+            ++nbad;
+            if (fix) indices[l + v] = static_cast<I>(0);
+          }
+        }
+      }
+    }
+  } else {  // a table boundary inside the block
+    for (int64_t base = p0; base < p1; base += 256 * kIdxPerThread) {
+      I idx[kIdxPerThread];
+#pragma unroll
+      for (int k = 0; k < kIdxPerThread; ++k) {
+        const int64_t l = base + k * 256 + tid;
+        idx[k] = l < p1 ? indices[l] : I(0);
+      }
+#pragma unroll
+      for (int k = 0; k < kIdxPerThread; ++k) {
+        const int64_t l = base + k * 256 + tid;
+        if (l >= p1) break;
+        int lo = 0, hi = nb;  // s_rep[lo] <= l < s_rep[hi]
+        while (hi - lo > 1) {
+          const int mid = (lo + hi) >> 1;
+          if (static_cast<int64_t>(s_rep[mid]) <= l)
+            lo = mid;
+          else
+            hi = mid;
+        }
+        const int64_t x = static_cast<int64_t>(idx[k]);
+        if (x < 0 || x >= s_lim[lo]) {
+          ++nbad;
+          if (fix) indices[l] = static_cast<I>(0);
+        }
       }
     }
   }
@@ -187,7 +229,7 @@ struct BoundsWs {
 
 BoundsWs carve_bounds(uint8_t* base, int64_t nbags) {
   BoundsWs w{};
-  int64_t tile = 256;
+  int64_t tile = nbags <= kOneTile ? kOneTile : 256;
   while (ceil_div(nbags, tile) > 1024) tile *= 2;
   w.tile = tile;
   w.ntiles = ceil_div(nbags > 0 ? nbags : 1, tile);
@@ -200,13 +242,17 @@ template <typename I>
 int run_bounds(const int64_t* rows, void* indices, void* offsets, int64_t nbags, int64_t B,
                const int32_t* B_offsets, int32_t T, int64_t N, int32_t mode,
                unsigned long long* warning, const BoundsWs& w, hipStream_t s) {
-  // Bags per block: about one pass of index loads (1024 positions) per block
-  // at the batch's mean pooling factor, between 32 and 256 bags.
+  // Bags per block: between 32 and 256, the most that leaves eight blocks per
+  // CU, or fewer where their positions pass one round of loads.
   int32_t bpb = kMaxBagsPerBlock;
-  while (bpb > 32 && bpb * N > 256 * kIdxPerThread * nbags) bpb >>= 1;
-  tile_max_kernel<I><<<dim3(static_cast<uint32_t>(ceil_div(w.ntiles, 4))), 256, 0, s>>>(
-      static_cast<const I*>(offsets), nbags, N, w.tile, w.ntiles, w.tilemax);
-  MX_LAUNCH_CHECK();
+  const int64_t round = 256 * kIdxPerThread * static_cast<int64_t>(16 / sizeof(I));
+  const int64_t fill = static_cast<int64_t>(num_cus()) * 8;
+  while (bpb > 32 && bpb * N > round * nbags && ceil_div(nbags, bpb) < fill) bpb >>= 1;
+  if (w.ntiles > 1) {  // one tile: the blocks read their offsets themselves
+    tile_max_kernel<I><<<dim3(static_cast<uint32_t>(ceil_div(w.ntiles, 4))), 256, 0, s>>>(
+        static_cast<const I*>(offsets), nbags, N, w.tile, w.ntiles, w.tilemax);
+    MX_LAUNCH_CHECK();
+  }
   bounds_main_kernel<I><<<dim3(static_cast<uint32_t>(ceil_div(nbags, bpb))), 256, 0, s>>>(
       rows, static_cast<I*>(indices), static_cast<I*>(offsets), nbags, B, B_offsets, T, N, mode,
       warning, w.tilemax, w.tile, bpb);
