@@ -111,6 +111,40 @@ def test_nbit_nobag(dev, ty, out_dtype, D):
     np.testing.assert_array_equal(g, exp.view(np.uint32) if kind == 0 else exp.view(np.uint16))
 
 
+@pytest.mark.parametrize("ty", ALL_TYPES)
+@pytest.mark.parametrize("D", [4, 12, 56, 72, 100, 260, 516])
+def test_nbit_nobag_partial_blocks(dev, ty, D):
+    """Widths that leave a partial 8-element block, and each count of lanes per
+    position; more positions than one round of the grid's first block."""
+    print(f"[case] nbit nobag partial ty={ty} D={D}", flush=True)
+    rng = np.random.default_rng(ty * 31 + D)
+    rows = [33, 7, 50]
+    inp = random_tbe(rng, 3, 41, [D] * 3, rows, 25, empty_frac=0.2)
+    tys = [ty] * 3
+    buf, w_off = build_weights(rng, tys, [D] * 3, rows)
+    for out_dtype, kind in ((1, 1), (5, 2), (0, 0)):
+        got = _nbit_nobag(dev, buf, w_off, tys, D, inp, out_dtype).cpu()
+        exp = orc.nbit_forward_nobag(buf, w_off, tys, D, inp.B, inp.indices, inp.offsets,
+                                     out_kind=kind)
+        g = got.view(torch.int16).numpy() if kind else got.numpy().view(np.uint32)
+        np.testing.assert_array_equal(g.view(np.uint16 if kind else np.uint32),
+                                      exp.view(np.uint16 if kind else np.uint32))
+
+
+def test_nbit_nobag_many_tables(dev):
+    """More tables than the first positions kept in LDS (1024)."""
+    print("[case] nbit nobag T=1100", flush=True)
+    rng = np.random.default_rng(17)
+    T, D = 1100, 16
+    tys = [orc.INT8 if t % 3 else orc.INT4 for t in range(T)]
+    rows = [int(x) for x in rng.integers(1, 6, T)]
+    inp = random_tbe(rng, T, 2, [D] * T, rows, 4, empty_frac=0.3)
+    buf, w_off = build_weights(rng, tys, [D] * T, rows)
+    got = _nbit_nobag(dev, buf, w_off, tys, D, inp, 1)
+    exp = orc.nbit_forward_nobag(buf, w_off, tys, D, inp.B, inp.indices, inp.offsets, out_kind=1)
+    np.testing.assert_array_equal(got.cpu().numpy().view(np.uint16), exp.view(np.uint16))
+
+
 def test_nbit_nobag_mixed_types(dev):
     """Tables of all six types in one call (one launch per type)."""
     print("[case] nbit nobag mixed types", flush=True)
