@@ -515,6 +515,21 @@ int mx_permute_2d_data(const int32_t* permute, int64_t T_out, int32_t T, int64_t
                        int64_t in_len, const float* weights, int64_t out_len,
                        void* permuted_indices, float* permuted_weights, void* stream);
 
+/* The same op for a batch of few features (at most 1024 in and out), without
+ * the cumsums: mx_permute_2d_workspace_bytes gives the bytes of the features'
+ * sums, or 0 where only the two steps above serve the batch.
+ * mx_permute_2d_sums writes the permuted lengths and the sums (and the permuted
+ * lengths' sum to the device word `total` unless null); mx_permute_2d_copy then
+ * copies indices (and weights) of in_len entries into out_len entries. */
+size_t mx_permute_2d_workspace_bytes(int64_t T_out, int32_t T, int64_t B);
+int mx_permute_2d_sums(const int32_t* permute, int64_t T_out, const void* lengths,
+                       int32_t length_bytes, int32_t T, int64_t B, void* permuted_lengths,
+                       void* workspace, size_t workspace_bytes, int64_t* total, void* stream);
+int mx_permute_2d_copy(const int32_t* permute, int64_t T_out, int32_t T, int64_t B,
+                       const void* workspace, const void* indices, int32_t index_bytes,
+                       int64_t in_len, const float* weights, int64_t out_len,
+                       void* permuted_indices, float* permuted_weights, void* stream);
+
 /* Serves fbgemm::offsets_range: out[j] = j - offsets[i] for j in segment i =
  * [offsets[i], offsets[i + 1]) (the last segment ends at range_size); out
  * [range_size], int32 or int64 like offsets. */

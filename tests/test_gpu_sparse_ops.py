@@ -164,3 +164,30 @@ def test_permute_2d_sparse_data_sizes(dev, T, B, Tp, ldtype):
     np.testing.assert_array_equal(pl.cpu().numpy(), exp_l)
     np.testing.assert_array_equal(pi.cpu().numpy(), exp_i)
     assert pw is None
+
+
+@pytest.mark.parametrize("T,Tp,B,maxlen", [(1, 1, 1, 40), (40, 40, 100, 30), (1024, 1024, 3, 5),
+                                           (1025, 1024, 3, 5), (300, 1025, 2, 5), (5, 7, 8192, 4),
+                                           (5, 7, 8193, 4), (2, 3, 40000, 3)])
+@pytest.mark.parametrize("idtype", [torch.int32, torch.int64])
+def test_permute_2d_by_feature(dev, T, Tp, B, maxlen, idtype):
+    """Either side of the feature counts and bag parts at which the per-feature
+    sums take over from the cumsums, blocks inside one feature and over many
+    short ones, and a given output size below the lengths' sum."""
+    print(f"[case] permute_2D by feature T={T} Tp={Tp} B={B} i={idtype}", flush=True)
+    rng = np.random.default_rng(T * 31 + B)
+    lengths = rng.integers(0, maxlen, (T, B))
+    lengths[rng.random(T) < 0.2] = 0
+    n = int(lengths.sum())
+    idx, w = rng.integers(0, 10**6, n), rng.standard_normal(n).astype(np.float32)
+    permute = rng.integers(0, T, Tp).astype(np.int32)
+    exp_l, exp_i, exp_w = orc.permute_2d_sparse_data(permute, lengths, idx, w)
+    args = (torch.from_numpy(permute).to(dev), torch.from_numpy(lengths).to(dev),
+            torch.from_numpy(idx).to(dev, idtype), torch.from_numpy(w).to(dev))
+    cut = exp_i.size - exp_i.size // 3
+    for size in (None, exp_i.size, cut):
+        pl, pi, pw = torch.ops.fbgemm.permute_2D_sparse_data(*args, size)
+        m = exp_i.size if size is None else size
+        np.testing.assert_array_equal(pl.cpu().numpy(), exp_l)
+        np.testing.assert_array_equal(pi.cpu().numpy(), exp_i[:m])
+        np.testing.assert_array_equal(pw.cpu().numpy(), exp_w[:m])

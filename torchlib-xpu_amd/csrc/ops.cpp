@@ -1832,13 +1832,29 @@ std::tuple<Tensor, Tensor, std::optional<Tensor>> permute_2D_sparse_data(
   const Tensor perm = permute.contiguous(), len = lengths.contiguous(), idx = indices.contiguous();
   const int32_t lb = static_cast<int32_t>(len.element_size());
   Tensor plen = at::empty({Tp, B}, len.options());
-  MX_CALL(mx_permute_2d_lengths(perm.data_ptr<int32_t>(), Tp, len.data_ptr(), lb,
-                                static_cast<int32_t>(T), B, plen.data_ptr(), stream_of(len)));
-  const Tensor in_off = cumsum_impl(len.view({-1}), 2);
-  const Tensor out_off = cumsum_impl(plen.view({-1}), 2);
-  const int64_t out_len = permuted_lengths_sum.has_value()
-                              ? permuted_lengths_sum->expect_int()
-                              : out_off[Tp * B].item<int64_t>();  // one host sync, as upstream
+  // Few features: their sums alone place the data; else both complete cumsums.
+  const size_t ws_bytes = mx_permute_2d_workspace_bytes(Tp, static_cast<int32_t>(T), B);
+  Tensor in_off, out_off, sums;
+  int64_t out_len = 0;
+  if (ws_bytes > 0) {
+    const int64_t words = static_cast<int64_t>(ws_bytes / sizeof(int64_t));
+    sums = at::empty({words + 1}, len.options().dtype(at::kLong));  // + the total
+    int64_t* total = sums.data_ptr<int64_t>() + words;
+    MX_CALL(mx_permute_2d_sums(perm.data_ptr<int32_t>(), Tp, len.data_ptr(), lb,
+                               static_cast<int32_t>(T), B, plen.data_ptr(), sums.data_ptr(),
+                               ws_bytes, permuted_lengths_sum.has_value() ? nullptr : total,
+                               stream_of(len)));
+    out_len = permuted_lengths_sum.has_value() ? permuted_lengths_sum->expect_int()
+                                               : sums[words].item<int64_t>();  // one host sync
+  } else {
+    MX_CALL(mx_permute_2d_lengths(perm.data_ptr<int32_t>(), Tp, len.data_ptr(), lb,
+                                  static_cast<int32_t>(T), B, plen.data_ptr(), stream_of(len)));
+    in_off = cumsum_impl(len.view({-1}), 2);
+    out_off = cumsum_impl(plen.view({-1}), 2);
+    out_len = permuted_lengths_sum.has_value()
+                  ? permuted_lengths_sum->expect_int()
+                  : out_off[Tp * B].item<int64_t>();  // one host sync, as upstream
+  }
   Tensor pidx = at::empty({out_len}, idx.options());
   std::optional<Tensor> pw;
   Tensor wc;
@@ -1848,6 +1864,14 @@ std::tuple<Tensor, Tensor, std::optional<Tensor>> permute_2D_sparse_data(
                 "weights must be fp32 with one entry per index");
     wc = weights->contiguous();
     pw = at::empty({out_len}, wc.options());
+  }
+  if (ws_bytes > 0) {
+    MX_CALL(mx_permute_2d_copy(perm.data_ptr<int32_t>(), Tp, static_cast<int32_t>(T), B,
+                               sums.data_ptr(), idx.data_ptr(), ib, idx.numel(),
+                               wc.defined() ? wc.data_ptr<float>() : nullptr, out_len,
+                               pidx.data_ptr(), pw.has_value() ? pw->data_ptr<float>() : nullptr,
+                               stream_of(len)));
+    return {plen, pidx, pw};
   }
   MX_CALL(mx_permute_2d_data(perm.data_ptr<int32_t>(), Tp, static_cast<int32_t>(T), B,
                              in_off.data_ptr(), out_off.data_ptr(), lb, idx.data_ptr(), ib,

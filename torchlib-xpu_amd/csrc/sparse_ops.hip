@@ -25,8 +25,15 @@
 // scans its tile from its prefix, the sum of the tiles before it (added up by
 // the block itself up to 1024 tiles, beyond that scanned first by one block;
 // a batch of one tile takes only the last launch).  A 2-D complete cumsum gives each
-// row to one block.  The permute copies each output bag with one 16-lane
-// group (consecutive elements, coalesced), from the two complete cumsums.
+// row to one block.  A permute keeps the order of a feature's bags, so each
+// output feature is one contiguous copy of an input feature, and only the
+// features' sums and their prefixes are needed: one launch sums each feature's
+// lengths and copies the permuted lengths, a second copies the data, each of
+// its blocks building the prefixes in LDS.  (40 features x 4096 bags, 1.6M
+// int64 indices with weights, the new offsets' cumsum included: 50 us with a
+// permute launch, two cumsums and a copy per bag, 27 this way; 3 x 16 bags 28.5
+// -> 18.3, 800 x 16 bags 37 -> 31.)  Batches of more than kPermMaxT features take that longer
+// way: one 16-lane group per output bag, from the two complete cumsums.
 #include <type_traits>
 
 #include "mx_common.h"
@@ -259,6 +266,215 @@ __global__ void __launch_bounds__(256)
   }
 }
 
+// Features whose sums fit a block's LDS, lengths summed per block, and the sums
+// a block of the copy adds up itself.
+constexpr int64_t kPermMaxT = 1024;
+constexpr int64_t kPermPart = 8192;
+constexpr int64_t kPermMaxSums = 8192;
+
+int64_t perm_parts(int64_t B) { return ceil_div(B, kPermPart); }
+
+bool perm_by_feature(int64_t T, int64_t Tp, int64_t B) {
+  return T >= 1 && T <= kPermMaxT && Tp >= 1 && Tp <= kPermMaxT && B >= 1 &&
+         T * perm_parts(B) <= kPermMaxSums;
+}
+
+// Blocks [0, T * parts): the sum of part p of feature t's lengths.  The blocks
+// after them: the permuted lengths, part p of output feature f.
+template <typename L>
+__global__ void __launch_bounds__(kCsThreads)
+    permute_sums_kernel(const int32_t* __restrict__ permute, const L* __restrict__ lengths,
+                        int32_t T, int64_t B, int32_t parts, L* __restrict__ out,
+                        int64_t* __restrict__ sums) {
+  const int64_t bid = blockIdx.x, nsum = static_cast<int64_t>(T) * parts;
+  const bool sum = bid < nsum;  // block-uniform
+  const int64_t x = sum ? bid : bid - nsum;
+  const int64_t f = x / parts, b0 = (x - f * parts) * kPermPart;
+  const int64_t b1 = b0 + kPermPart < B ? b0 + kPermPart : B;
+  const int64_t src = sum ? f : static_cast<int64_t>(permute[f]);
+  const bool valid = src >= 0 && src < T;
+  L v[kPermPart / kCsThreads];
+  int64_t s = 0;
+#pragma unroll
+  for (int it = 0; it < kPermPart / kCsThreads; ++it) {
+    const int64_t b = b0 + it * kCsThreads + threadIdx.x;
+    v[it] = valid && b < b1 ? lengths[src * B + b] : L(0);
+    s += static_cast<int64_t>(v[it]);
+  }
+  if (sum) {
+    int64_t total;
+    (void)block_excl<int64_t>(s, &total);
+    if (threadIdx.x == 0) sums[bid] = total;
+    return;
+  }
+#pragma unroll
+  for (int it = 0; it < kPermPart / kCsThreads; ++it) {
+    const int64_t b = b0 + it * kCsThreads + threadIdx.x;
+    if (b < b1) out[f * B + b] = v[it];
+  }
+}
+
+constexpr int kPermThreads = 256;
+constexpr int kPermOwn = kPermMaxT / kPermThreads;  // features per thread in the prefixes
+
+// start[i] = val[0] + ... + val[i-1] for i <= n (n <= kPermMaxT), in LDS.
+__device__ __forceinline__ void perm_starts(const int64_t* val, int32_t n, int64_t* start) {
+  __shared__ int64_t wsum[kPermThreads / 64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int32_t i0 = threadIdx.x * kPermOwn;
+  int64_t own = 0;
+#pragma unroll
+  for (int i = 0; i < kPermOwn; ++i) own += i0 + i < n ? val[i0 + i] : 0;
+  int64_t incl = own;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int64_t o = __shfl_up(incl, d, 64);
+    if (lane >= d) incl += o;
+  }
+  if (lane == 63) wsum[w] = incl;
+  __syncthreads();
+  int64_t at = incl - own;
+  for (int i = 0; i < w; ++i) at += wsum[i];
+#pragma unroll
+  for (int i = 0; i < kPermOwn; ++i)
+    if (i0 + i < n) {
+      start[i0 + i] = at;
+      at += val[i0 + i];
+      if (i0 + i == n - 1) start[n] = at;
+    }
+  __syncthreads();
+}
+
+struct PermPrefixes {
+  int64_t val[kPermMaxT];        // a feature's sum, input then output
+  int64_t in[kPermMaxT + 1];     // first index of each input feature
+  int64_t out[kPermMaxT + 1];    // first index of each output feature
+};
+
+__device__ __forceinline__ void perm_prefixes(const int32_t* __restrict__ permute, int32_t T,
+                                              int32_t Tp, int32_t parts,
+                                              const int64_t* __restrict__ sums, PermPrefixes& m) {
+  for (int32_t t = threadIdx.x; t < T; t += kPermThreads) {
+    int64_t s = 0;
+    for (int32_t p = 0; p < parts; ++p) s += sums[static_cast<int64_t>(t) * parts + p];
+    m.val[t] = s;
+  }
+  __syncthreads();
+  perm_starts(m.val, T, m.in);
+  int64_t mine[kPermOwn];
+#pragma unroll
+  for (int i = 0; i < kPermOwn; ++i) {
+    const int32_t f = i * kPermThreads + static_cast<int32_t>(threadIdx.x);
+    const int32_t src = f < Tp ? permute[f] : -1;
+    mine[i] = src >= 0 && src < T ? m.val[src] : 0;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kPermOwn; ++i) {
+    const int32_t f = i * kPermThreads + static_cast<int32_t>(threadIdx.x);
+    if (f < Tp) m.val[f] = mine[i];
+  }
+  __syncthreads();
+  perm_starts(m.val, Tp, m.out);
+}
+
+// The permuted lengths' sum (the output's size).
+__global__ void __launch_bounds__(kPermThreads)
+    permute_total_kernel(const int32_t* __restrict__ permute, int32_t T, int32_t Tp, int32_t parts,
+                         const int64_t* __restrict__ sums, int64_t* __restrict__ total) {
+  __shared__ PermPrefixes m;
+  perm_prefixes(permute, T, Tp, parts, sums, m);
+  if (threadIdx.x == 0) *total = m.out[Tp];
+}
+
+// Copies out[o0, o1) from in + (s0 - o0): 16 bytes per thread and step, at the
+// element type's own alignment.
+template <typename E>
+__device__ __forceinline__ void perm_copy(const E* __restrict__ in, E* __restrict__ out,
+                                          int64_t o0, int64_t o1, int64_t shift) {
+  constexpr int V = 16 / sizeof(E), K = 4;
+  typedef E EV __attribute__((ext_vector_type(V), aligned(sizeof(E))));
+  for (int64_t base = o0; base < o1; base += kPermThreads * V * K) {
+    EV x[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int64_t o = base + (k * kPermThreads + static_cast<int64_t>(threadIdx.x)) * V;
+      if (o + V <= o1) {
+        x[k] = *reinterpret_cast<const EV*>(in + o + shift);
+      } else {
+#pragma unroll
+        for (int v = 0; v < V; ++v) x[k][v] = o + v < o1 ? in[o + v + shift] : E(0);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int64_t o = base + (k * kPermThreads + static_cast<int64_t>(threadIdx.x)) * V;
+      if (o + V <= o1) {
+        *reinterpret_cast<EV*>(out + o) = x[k];
+      } else {
+#pragma unroll
+        for (int v = 0; v < V; ++v)
+          if (o + v < o1) out[o + v] = x[k][v];
+      }
+    }
+  }
+}
+
+// A block copies the output's indices [blockIdx * chunk, + chunk): the parts of
+// the output features it meets, one contiguous copy each where they are long,
+// else element by element, each finding its feature in the prefixes.  Lengths
+// that disagree with the index count or the given output size stop the copy
+// instead of reading or writing past either array.
+template <typename I>
+__global__ void __launch_bounds__(kPermThreads)
+    permute_copy_kernel(const int32_t* __restrict__ permute, int32_t T, int32_t Tp, int32_t parts,
+                        const int64_t* __restrict__ sums, const I* __restrict__ indices,
+                        const float* __restrict__ weights, int64_t in_len, int64_t chunk,
+                        I* __restrict__ out_indices, float* __restrict__ out_weights,
+                        int64_t out_len) {
+  __shared__ PermPrefixes m;
+  perm_prefixes(permute, T, Tp, parts, sums, m);
+  const int64_t total = m.out[Tp] < out_len ? m.out[Tp] : out_len;
+  const int64_t c0 = blockIdx.x * chunk, c1 = c0 + chunk < total ? c0 + chunk : total;
+  if (c0 >= c1) return;  // block-uniform
+  auto feature = [&](int64_t o) {  // the last f with out[f] <= o
+    int32_t lo = 0, hi = Tp;
+    while (hi - lo > 1) {
+      const int32_t mid = lo + ((hi - lo) >> 1);
+      if (m.out[mid] <= o)
+        lo = mid;
+      else
+        hi = mid;
+    }
+    return lo;
+  };
+  const int32_t f0 = feature(c0), f1 = feature(c1 - 1);
+  if (f1 - f0 < 4) {  // block-uniform: long features
+    for (int32_t f = f0; f <= f1; ++f) {
+      const int32_t src = permute[f];
+      if (src < 0 || src >= T) continue;  // its length is 0
+      const int64_t s0 = m.in[src], d0 = m.out[f];
+      if (s0 < 0 || d0 < 0) continue;  // negative lengths upstream: nothing in bounds to copy
+      const int64_t shift = s0 - d0;
+      const int64_t o0 = c0 > d0 ? c0 : d0;
+      int64_t o1 = m.out[f + 1] < c1 ? m.out[f + 1] : c1;
+      o1 = o1 < in_len - shift ? o1 : in_len - shift;
+      if (o0 >= o1) continue;
+      perm_copy<I>(indices, out_indices, o0, o1, shift);
+      if (weights) perm_copy<float>(weights, out_weights, o0, o1, shift);
+    }
+    return;
+  }
+  for (int64_t o = c0 + threadIdx.x; o < c1; o += kPermThreads) {
+    const int32_t f = feature(o), src = permute[f];
+    if (src < 0 || src >= T || m.in[src] < 0 || m.out[f] < 0) continue;
+    const int64_t i = m.in[src] + (o - m.out[f]);
+    if (i < 0 || i >= in_len) continue;
+    out_indices[o] = indices[i];
+    if (weights) out_weights[o] = weights[i];
+  }
+}
+
 // A 16-lane group per segment writes j - start over its range.
 template <typename I>
 __global__ void __launch_bounds__(256)
@@ -411,6 +627,76 @@ extern "C" int mx_permute_2d_data(const int32_t* permute, int64_t T_out, int32_t
       MX_PERM(int32_t, int32_t);
   }
 #undef MX_PERM
+  MX_LAUNCH_CHECK();
+  return MX_OK;
+}
+
+extern "C" size_t mx_permute_2d_workspace_bytes(int64_t T_out, int32_t T, int64_t B) {
+  if (!perm_by_feature(T, T_out, B)) return 0;
+  return static_cast<size_t>(T * perm_parts(B)) * sizeof(int64_t);
+}
+
+extern "C" int mx_permute_2d_sums(const int32_t* permute, int64_t T_out, const void* lengths,
+                                  int32_t length_bytes, int32_t T, int64_t B,
+                                  void* permuted_lengths, void* workspace,
+                                  size_t workspace_bytes, int64_t* total, void* stream) {
+  clear_error();
+  MX_REQUIRE(length_bytes == 4 || length_bytes == 8, "lengths must be int32 or int64");
+  MX_REQUIRE(T >= 0 && B >= 0 && T_out >= 0, "negative size");
+  MX_REQUIRE(perm_by_feature(T, T_out, B), "too many features (or none) for sums per feature");
+  MX_REQUIRE(permute && permuted_lengths && lengths, "null pointer argument");
+  const size_t need = mx_permute_2d_workspace_bytes(T_out, T, B);
+  if (workspace == nullptr || workspace_bytes < need)
+    return set_error(MX_EWORKSPACE, "workspace of %zu bytes needed", need);
+  auto* s = as_stream(stream);
+  const int32_t parts = static_cast<int32_t>(perm_parts(B));
+  const dim3 gd(static_cast<uint32_t>((T + T_out) * parts));
+  auto* sums = static_cast<int64_t*>(workspace);
+  if (length_bytes == 8)
+    permute_sums_kernel<int64_t><<<gd, kCsThreads, 0, s>>>(
+        permute, static_cast<const int64_t*>(lengths), T, B, parts,
+        static_cast<int64_t*>(permuted_lengths), sums);
+  else
+    permute_sums_kernel<int32_t><<<gd, kCsThreads, 0, s>>>(
+        permute, static_cast<const int32_t*>(lengths), T, B, parts,
+        static_cast<int32_t*>(permuted_lengths), sums);
+  MX_LAUNCH_CHECK();
+  if (total) {
+    permute_total_kernel<<<1, kPermThreads, 0, s>>>(permute, T, static_cast<int32_t>(T_out), parts,
+                                                    sums, total);
+    MX_LAUNCH_CHECK();
+  }
+  return MX_OK;
+}
+
+extern "C" int mx_permute_2d_copy(const int32_t* permute, int64_t T_out, int32_t T, int64_t B,
+                                  const void* workspace, const void* indices, int32_t index_bytes,
+                                  int64_t in_len, const float* weights, int64_t out_len,
+                                  void* permuted_indices, float* permuted_weights,
+                                  void* stream) {
+  clear_error();
+  MX_REQUIRE(index_bytes == 4 || index_bytes == 8, "indices must be int32 or int64");
+  MX_REQUIRE(T >= 0 && B >= 0 && T_out >= 0 && out_len >= 0 && in_len >= 0, "negative size");
+  MX_REQUIRE(perm_by_feature(T, T_out, B), "too many features (or none) for sums per feature");
+  MX_REQUIRE(!weights == !permuted_weights, "weights and permuted_weights go together");
+  if (out_len == 0) return MX_OK;
+  MX_REQUIRE(permute && workspace && indices && permuted_indices, "null pointer argument");
+  auto* s = as_stream(stream);
+  // At least 2048 indices per block, and no more than eight blocks per CU, whose
+  // prefixes cost more than a copy of that size.
+  const int64_t cap = static_cast<int64_t>(num_cus()) * 8;
+  const int64_t chunk = ceil_div(ceil_div(out_len, cap), 2048) * 2048;
+  const dim3 gd(static_cast<uint32_t>(ceil_div(out_len, chunk)));
+  const int32_t parts = static_cast<int32_t>(perm_parts(B)), Tp = static_cast<int32_t>(T_out);
+  const auto* sums = static_cast<const int64_t*>(workspace);
+  if (index_bytes == 8)
+    permute_copy_kernel<int64_t><<<gd, kPermThreads, 0, s>>>(
+        permute, T, Tp, parts, sums, static_cast<const int64_t*>(indices), weights, in_len, chunk,
+        static_cast<int64_t*>(permuted_indices), permuted_weights, out_len);
+  else
+    permute_copy_kernel<int32_t><<<gd, kPermThreads, 0, s>>>(
+        permute, T, Tp, parts, sums, static_cast<const int32_t*>(indices), weights, in_len, chunk,
+        static_cast<int32_t*>(permuted_indices), permuted_weights, out_len);
   MX_LAUNCH_CHECK();
   return MX_OK;
 }
