@@ -84,6 +84,36 @@ def test_jagged_dense_add(dev, dtype, lengths, max_L, D):
     _bits_equal(got, exp)
 
 
+@pytest.mark.parametrize("dims", [1, 2, 3, 4])
+@pytest.mark.parametrize("max_L,D", [(3, 4), (16, 16), (17, 16), (64, 16), (65, 16), (300, 20),
+                                     (5, 3)])
+def test_bag_group_sizes(dev, dims, max_L, D):
+    """Chunks per innermost list either side of each group size (16, 64, 256
+    threads) and past one round, 1 to 4 jagged dims, truncated and empty lists,
+    values rows before the first list and past the last."""
+    print(f"[case] jagged groups dims={dims} max_L={max_L} D={D}", flush=True)
+    rng = np.random.default_rng(dims * 1000 + max_L + D)
+    offs, maxs, n = [], [], 7
+    for k in range(dims):
+        top = max_L if k == dims - 1 else 3
+        offs.append(_offsets(rng.integers(0, top + 3, n)))
+        maxs.append(top)
+        n = int(offs[-1][-1])
+    vals = rng.standard_normal((n, D)).astype(np.float32)
+    ot = [torch.from_numpy(o).to(dev) for o in offs]
+    exp = orc.jagged_to_padded_dense(vals, offs, maxs, padding_value=2.5)
+    got = torch.ops.fbgemm.jagged_to_padded_dense(torch.from_numpy(vals).to(dev), ot, maxs, 2.5)
+    _bits_equal(got, exp)
+    dense = rng.standard_normal(exp.shape).astype(np.float32)
+    for extra in (0, 5):  # rows past the last list
+        back, _ = torch.ops.fbgemm.dense_to_jagged(torch.from_numpy(dense).to(dev), ot, n + extra)
+        _bits_equal(back[:n], orc.dense_to_jagged(dense, offs))
+        assert not back[n:].any()
+    added, _ = torch.ops.fbgemm.jagged_dense_elementwise_add_jagged_output(
+        torch.from_numpy(vals).to(dev), ot, torch.from_numpy(dense).to(dev))
+    _bits_equal(added, orc.jagged_dense_elementwise_add(vals, offs, dense, "f32"))
+
+
 def test_two_jagged_dims(dev):
     print("[case] j2pd/d2j two jagged dims", flush=True)
     rng = np.random.default_rng(4)

@@ -10,12 +10,15 @@
 //
 // Design: the ops are pure HBM streams.  One work item moves VEC bytes
 // (16 when the row size and pointers allow it), consecutive work items walk
-// a row, so every wave issues fully coalesced 1 KiB transactions.  With one
-// jagged dim (the common case) a bag is a contiguous copy: one block row per
-// bag, no per-item index arithmetic.  With more, the jagged coordinate of a
-// dense row is found by walking the offsets levels (dense -> jagged) or by a
-// binary search per level (jagged -> dense); the offsets are a few KB and
-// stay in L2.
+// a row, so every wave issues fully coalesced transactions.  The rows of one
+// innermost list (a "bag": with one jagged dim a batch element) lie together
+// on both sides, so a group of threads moves a whole bag with no per-item
+// index arithmetic; with more jagged dims the bag's place on the other side is
+// found once per bag, by walking the offsets levels (padded dense -> list) or
+// by a binary search per outer level (list -> padded dense).  A group is 16,
+// 64 or 256 threads by the bag's size.  (Two jagged dims, 256 x 20 x 50 x 64
+// bf16, against coordinates per chunk: padding 26.6 -> 11.3 us, back 14.3 ->
+// 11.0 by trace; the fp32 add 21.2 -> 15.6 us per call.)
 #include "mx_common.h"
 
 namespace mx {
@@ -38,22 +41,32 @@ __device__ __forceinline__ int64_t off_at(const JaggedMeta& m, int k, int64_t i)
   return static_cast<int64_t>(reinterpret_cast<const I*>(m.off[k])[i]);
 }
 
-// Dense row r (over B * prod(max_len)) -> jagged values row, or -1 for padding.
+// Innermost list of dense bag r (over B * prod(max_len of the outer dims)):
+// its first values row and its length, 0 for a list that is not there.
 template <typename I>
-__device__ int64_t dense_to_values_row(int64_t r, const JaggedMeta& m) {
-  int64_t coord[MX_MAX_JAGGED_DIM];
-  for (int k = m.ndim - 1; k >= 0; --k) {
-    coord[k] = r % m.max_len[k];
-    r /= m.max_len[k];
+__device__ __forceinline__ void dense_bag(int64_t r, const JaggedMeta& m, int64_t& begin,
+                                          int64_t& len) {
+  const int last = m.ndim - 1;
+  int64_t idx = r;
+  if (last > 0) {
+    int64_t coord[MX_MAX_JAGGED_DIM - 1];
+    for (int k = last - 1; k >= 0; --k) {
+      const int64_t q = idx / m.max_len[k];
+      coord[k] = idx - q * m.max_len[k];
+      idx = q;
+    }
+    for (int k = 0; k < last; ++k) {
+      const int64_t b = off_at<I>(m, k, idx);
+      const int64_t e = off_at<I>(m, k, idx + 1);
+      if (coord[k] >= e - b) {
+        begin = len = 0;
+        return;
+      }
+      idx = b + coord[k];
+    }
   }
-  int64_t idx = r;  // b
-  for (int k = 0; k < m.ndim; ++k) {
-    const int64_t begin = off_at<I>(m, k, idx);
-    const int64_t end = off_at<I>(m, k, idx + 1);
-    if (coord[k] >= end - begin) return -1;
-    idx = begin + coord[k];
-  }
-  return idx;
+  begin = off_at<I>(m, last, idx);
+  len = off_at<I>(m, last, idx + 1) - begin;
 }
 
 // Last p in [0, n-1) with off[p] <= x, or -1 when x is past the last offset.
@@ -72,59 +85,22 @@ __device__ int64_t owner_of(const JaggedMeta& m, int k, int64_t x) {
   return lo;
 }
 
-// Jagged values row i -> dense row, or -1 if it has no dense position.
+// Innermost list p -> its dense bag, or -1 if it has no dense position.
 template <typename I>
-__device__ int64_t values_to_dense_row(int64_t i, const JaggedMeta& m) {
-  int64_t coord[MX_MAX_JAGGED_DIM];
-  int64_t idx = i;
-  bool inside = true;
-  for (int k = m.ndim - 1; k >= 0; --k) {
-    const int64_t p = owner_of<I>(m, k, idx);
-    if (p < 0) return -1;
-    coord[k] = idx - off_at<I>(m, k, p);
-    if (coord[k] >= m.max_len[k]) inside = false;
-    idx = p;
+__device__ __forceinline__ int64_t list_dense_bag(int64_t p, const JaggedMeta& m) {
+  const int last = m.ndim - 1;
+  if (last == 0) return p;
+  int64_t coord[MX_MAX_JAGGED_DIM - 1];
+  int64_t idx = p;
+  for (int k = last - 1; k >= 0; --k) {
+    const int64_t q = owner_of<I>(m, k, idx);
+    if (q < 0) return -1;
+    coord[k] = idx - off_at<I>(m, k, q);
+    if (coord[k] >= m.max_len[k]) return -1;
+    idx = q;
   }
-  if (!inside) return -1;
-  int64_t r = idx;
-  for (int k = 0; k < m.ndim; ++k) r = r * m.max_len[k] + coord[k];
-  return r;
-}
-
-template <int VEC, typename I>
-__global__ void __launch_bounds__(256) j2pd_kernel(const uint8_t* __restrict__ values,
-                                                   uint8_t* __restrict__ out, JaggedMeta m,
-                                                   int64_t rows, int64_t vpr, Chunk<VEC> pad) {
-  const int64_t total = rows * vpr;
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
-  for (int64_t w = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; w < total;
-       w += stride) {
-    const int64_t r = w / vpr;
-    const int64_t v = w - r * vpr;
-    const int64_t src = dense_to_values_row<I>(r, m);
-    Chunk<VEC> c = pad;
-    if (src >= 0) c = reinterpret_cast<const Chunk<VEC>*>(values)[src * vpr + v];
-    reinterpret_cast<Chunk<VEC>*>(out)[w] = c;
-  }
-}
-
-template <int VEC, typename I>
-__global__ void __launch_bounds__(256) d2j_kernel(const uint8_t* __restrict__ dense,
-                                                  uint8_t* __restrict__ out, JaggedMeta m,
-                                                  int64_t total_L, int64_t vpr) {
-  const int64_t total = total_L * vpr;
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
-  for (int64_t w = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; w < total;
-       w += stride) {
-    const int64_t i = w / vpr;
-    const int64_t v = w - i * vpr;
-    const int64_t dr = values_to_dense_row<I>(i, m);
-    Chunk<VEC> c;
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) c.b[e] = 0;
-    if (dr >= 0) c = reinterpret_cast<const Chunk<VEC>*>(dense)[dr * vpr + v];
-    reinterpret_cast<Chunk<VEC>*>(out)[w] = c;
-  }
+  for (int k = 0; k < last; ++k) idx = idx * m.max_len[k] + coord[k];
+  return idx;
 }
 
 // ---- element arithmetic for the jagged + dense add ------------------------
@@ -181,72 +157,57 @@ struct BinOp<MX_DTYPE_BF16, MUL> {
   }
 };
 
-template <int VEC, typename I, int DT, bool MUL>
-__global__ void __launch_bounds__(256) jagged_add_kernel(const uint8_t* __restrict__ x,
-                                                         const uint8_t* __restrict__ y,
-                                                         uint8_t* __restrict__ out, JaggedMeta m,
-                                                         int64_t total_L, int64_t vpr) {
-  using Op = BinOp<DT, MUL>;
-  const int64_t total = total_L * vpr;
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
-  for (int64_t w = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; w < total;
-       w += stride) {
-    const int64_t i = w / vpr;
-    const int64_t v = w - i * vpr;
-    const int64_t dr = values_to_dense_row<I>(i, m);
-    const Chunk<VEC> cx = reinterpret_cast<const Chunk<VEC>*>(x)[w];
-    Chunk<VEC> cy;
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) cy.b[e] = 0;  // +0 in every element type
-    if (dr >= 0) cy = reinterpret_cast<const Chunk<VEC>*>(y)[dr * vpr + v];
-    Chunk<VEC> co;
-#pragma unroll
-    for (int e = 0; e < VEC; e += Op::kBytes) Op::apply(cx.b + e, cy.b + e, co.b + e);
-    reinterpret_cast<Chunk<VEC>*>(out)[w] = co;
-  }
-}
-
-// ---- one jagged dimension: a bag is a contiguous copy ----------------------
+// ---- a bag is a contiguous copy ---------------------------------------------
 //
-// With a single jagged dim, bag b's values rows are [off[b], off[b+1]) and its
-// dense rows [b*max_L, (b+1)*max_L): both contiguous, so each bag is one
-// straight copy plus padding, with no per-chunk coordinate arithmetic.  Grid
-// (x = bag, y = part of the bag); every thread keeps kJagItems chunks in
-// flight.
+// Dense bag r's rows [r*max_L, (r+1)*max_L) and its list's values rows are both
+// contiguous, so each bag is one straight copy plus padding.  2^lg threads per
+// bag (x), parts of a bag in y; every thread keeps kJagItems chunks in flight.
+// ONE: one jagged dim and a block per bag, as constants (a large bf16 round
+// trip 103.6 -> 101.5 us, a small add 6.8 -> 6.1 us against run-time values).
 
 constexpr int kJagItems = 4;
-constexpr int64_t kJagSpan = 256 * kJagItems;
 
-template <int VEC, typename I>
+template <int VEC, typename I, bool ONE>
 __global__ void __launch_bounds__(256)
-    j2pd1_kernel(const uint8_t* __restrict__ values, uint8_t* __restrict__ out,
-                 const I* __restrict__ off, int64_t max_L, int64_t vpr, Chunk<VEC> pad) {
-  const int64_t b = blockIdx.x;
-  const int64_t begin = static_cast<int64_t>(off[b]);
-  int64_t len = static_cast<int64_t>(off[b + 1]) - begin;
-  len = len < 0 ? 0 : (len > max_L ? max_L : len);
-  const int64_t n_copy = len * vpr, n_all = max_L * vpr;
-  const Chunk<VEC>* __restrict__ src = reinterpret_cast<const Chunk<VEC>*>(values) + begin * vpr;
-  Chunk<VEC>* __restrict__ dst = reinterpret_cast<Chunk<VEC>*>(out) + b * n_all;
-  for (int64_t base = blockIdx.y * kJagSpan; base < n_all; base += gridDim.y * kJagSpan) {
-    Chunk<VEC> c[kJagItems];
+    j2pd_kernel(const uint8_t* __restrict__ values, uint8_t* __restrict__ out, JaggedMeta m,
+                int64_t nbags, int32_t lg, int64_t vpr, Chunk<VEC> pad) {
+  if constexpr (ONE) {
+    lg = 8;
+    m.ndim = 1;
+  }
+  const int32_t tpb = 1 << lg, t = threadIdx.x & (tpb - 1);
+  const int64_t max_L = m.max_len[m.ndim - 1];
+  const int64_t span = static_cast<int64_t>(tpb) * kJagItems;
+  const int64_t step = static_cast<int64_t>(gridDim.x) << (8 - lg);
+  for (int64_t b = (static_cast<int64_t>(blockIdx.x) << (8 - lg)) + (threadIdx.x >> lg); b < nbags;
+       b += step) {
+    int64_t begin, len;
+    dense_bag<I>(b, m, begin, len);
+    len = len < 0 ? 0 : (len > max_L ? max_L : len);
+    const int64_t n_copy = len * vpr, n_all = max_L * vpr;
+    const Chunk<VEC>* __restrict__ src =
+        reinterpret_cast<const Chunk<VEC>*>(values) + begin * vpr;
+    Chunk<VEC>* __restrict__ dst = reinterpret_cast<Chunk<VEC>*>(out) + b * n_all;
+    for (int64_t base = blockIdx.y * span; base < n_all; base += gridDim.y * span) {
+      Chunk<VEC> c[kJagItems];
 #pragma unroll
-    for (int it = 0; it < kJagItems; ++it) {
-      const int64_t i = base + it * 256 + threadIdx.x;
-      c[it] = i < n_copy ? src[i] : pad;
-    }
+      for (int it = 0; it < kJagItems; ++it) {
+        const int64_t i = base + it * tpb + t;
+        c[it] = i < n_copy ? src[i] : pad;
+      }
 #pragma unroll
-    for (int it = 0; it < kJagItems; ++it) {
-      const int64_t i = base + it * 256 + threadIdx.x;
-      if (i < n_all) {
-        // The dense output streams past the caches (config 1 cold round trip
-        // 12.4 -> 11.8 us; the same for dense_to_jagged's output gained nothing).
-        if constexpr (VEC == 16) {
-          typedef unsigned int u4nt __attribute__((ext_vector_type(4)));
-          __builtin_nontemporal_store(*reinterpret_cast<const u4nt*>(&c[it]),
-                                      reinterpret_cast<u4nt*>(&dst[i]));
-        } else {
-          dst[i] = c[it];
+      for (int it = 0; it < kJagItems; ++it) {
+        const int64_t i = base + it * tpb + t;
+        if (i < n_all) {
+          // The dense output streams past the caches (config 1 cold round trip
+          // 12.4 -> 11.8 us; the same for dense_to_jagged's output gained nothing).
+          if constexpr (VEC == 16) {
+            typedef unsigned int u4nt __attribute__((ext_vector_type(4)));
+            __builtin_nontemporal_store(*reinterpret_cast<const u4nt*>(&c[it]),
+                                        reinterpret_cast<u4nt*>(&dst[i]));
+          } else {
+            dst[i] = c[it];
+          }
         }
       }
     }
@@ -260,16 +221,19 @@ template <int VEC, bool ADD, int DT, bool MUL>
 __device__ __forceinline__ void emit_rows(const uint8_t* __restrict__ dense,
                                           const uint8_t* __restrict__ x,
                                           uint8_t* __restrict__ out, int64_t r0, int64_t r1,
-                                          int64_t copy_rows, int64_t dense_row0, int64_t vpr) {
+                                          int64_t copy_rows, int64_t dense_row0, int64_t vpr,
+                                          int32_t tpb) {
+  const int32_t t = threadIdx.x & (tpb - 1);
+  const int64_t span = static_cast<int64_t>(tpb) * kJagItems;
   const int64_t n_all = (r1 - r0) * vpr, n_copy = copy_rows * vpr;
   const Chunk<VEC>* __restrict__ src = reinterpret_cast<const Chunk<VEC>*>(dense) + dense_row0 * vpr;
   Chunk<VEC>* __restrict__ dst = reinterpret_cast<Chunk<VEC>*>(out) + r0 * vpr;
   const Chunk<VEC>* __restrict__ xs = reinterpret_cast<const Chunk<VEC>*>(x) + r0 * vpr;
-  for (int64_t base = blockIdx.y * kJagSpan; base < n_all; base += gridDim.y * kJagSpan) {
+  for (int64_t base = blockIdx.y * span; base < n_all; base += gridDim.y * span) {
     Chunk<VEC> y[kJagItems];
 #pragma unroll
     for (int it = 0; it < kJagItems; ++it) {
-      const int64_t i = base + it * 256 + threadIdx.x;
+      const int64_t i = base + it * tpb + t;
       if (i < n_copy) {
         y[it] = src[i];
       } else {
@@ -279,7 +243,7 @@ __device__ __forceinline__ void emit_rows(const uint8_t* __restrict__ dense,
     }
 #pragma unroll
     for (int it = 0; it < kJagItems; ++it) {
-      const int64_t i = base + it * 256 + threadIdx.x;
+      const int64_t i = base + it * tpb + t;
       if (i >= n_all) continue;
       if constexpr (ADD) {
         const Chunk<VEC> cx = xs[i];
@@ -295,38 +259,63 @@ __device__ __forceinline__ void emit_rows(const uint8_t* __restrict__ dense,
   }
 }
 
-// Block x < nbags: bag x.  Block x == nbags: the values rows no bag covers
-// (before off[0], from off[nbags] on), which have no dense position.  Row
-// ranges are clamped to [0, total_L], so malformed offsets never write out
-// of bounds.
-template <int VEC, typename I, bool ADD, int DT, bool MUL>
+// Group x < nlists: innermost list x.  Group x == nlists: the values rows no
+// list covers (before the first offset, from the last on), which have no dense
+// position.  Row ranges are clamped to [0, total_L], so malformed offsets never
+// write out of bounds.
+template <int VEC, typename I, bool ADD, int DT, bool MUL, bool ONE>
 __global__ void __launch_bounds__(256)
-    jagged_out1_kernel(const uint8_t* __restrict__ dense, const uint8_t* __restrict__ x,
-                       uint8_t* __restrict__ out, const I* __restrict__ off, int64_t nbags,
-                       int64_t max_L, int64_t total_L, int64_t vpr) {
+    jagged_out_kernel(const uint8_t* __restrict__ dense, const uint8_t* __restrict__ x,
+                      uint8_t* __restrict__ out, JaggedMeta m, int64_t nlists, int32_t lg,
+                      int64_t total_L, int64_t vpr) {
+  if constexpr (ONE) {
+    lg = 8;
+    m.ndim = 1;
+  }
   auto clamp = [&](int64_t v, int64_t lo) { return v < lo ? lo : (v > total_L ? total_L : v); };
-  const int64_t b = blockIdx.x;
-  if (b < nbags) {
-    const int64_t r0 = clamp(static_cast<int64_t>(off[b]), 0);
-    const int64_t r1 = clamp(static_cast<int64_t>(off[b + 1]), r0);
-    const int64_t copy = r1 - r0 < max_L ? r1 - r0 : max_L;
-    emit_rows<VEC, ADD, DT, MUL>(dense, x, out, r0, r1, copy, b * max_L, vpr);
-  } else {
-    const int64_t head = clamp(static_cast<int64_t>(off[0]), 0);
-    const int64_t tail = clamp(static_cast<int64_t>(off[nbags]), head);
-    emit_rows<VEC, ADD, DT, MUL>(dense, x, out, 0, head, 0, 0, vpr);
-    emit_rows<VEC, ADD, DT, MUL>(dense, x, out, tail, total_L, 0, 0, vpr);
+  const int last = m.ndim - 1;
+  const int64_t max_L = m.max_len[last];
+  const int32_t tpb = 1 << lg;
+  const int64_t step = static_cast<int64_t>(gridDim.x) << (8 - lg);
+  for (int64_t p = (static_cast<int64_t>(blockIdx.x) << (8 - lg)) + (threadIdx.x >> lg);
+       p <= nlists; p += step) {
+    if (p < nlists) {
+      const int64_t r0 = clamp(off_at<I>(m, last, p), 0);
+      const int64_t r1 = clamp(off_at<I>(m, last, p + 1), r0);
+      if (r1 == r0) continue;
+      const int64_t bag = list_dense_bag<I>(p, m);
+      const int64_t copy = bag < 0 ? 0 : (r1 - r0 < max_L ? r1 - r0 : max_L);
+      emit_rows<VEC, ADD, DT, MUL>(dense, x, out, r0, r1, copy, bag < 0 ? 0 : bag * max_L, vpr,
+                                   tpb);
+    } else {
+      const int64_t head = clamp(off_at<I>(m, last, 0), 0);
+      const int64_t tail = clamp(off_at<I>(m, last, nlists), head);
+      emit_rows<VEC, ADD, DT, MUL>(dense, x, out, 0, head, 0, 0, vpr, tpb);
+      emit_rows<VEC, ADD, DT, MUL>(dense, x, out, tail, total_L, 0, 0, vpr, tpb);
+    }
   }
 }
 
 // ---- host side ------------------------------------------------------------
 
-// Grid of the single-jagged-dim kernels: one x per bag (plus extra), parts
-// of a bag in y.
-dim3 grid_1d(int64_t bags, int64_t chunks_per_bag) {
-  int64_t parts = ceil_div(chunks_per_bag > 0 ? chunks_per_bag : 1, kJagSpan);
-  if (parts > 64) parts = 64;  // the kernels loop over the rest
-  return dim3(static_cast<uint32_t>(bags), static_cast<uint32_t>(parts));
+// Threads per bag (2^lg) and grid: the smallest group that holds a full bag's
+// chunks in one round, kJagItems per thread, up to a block; bags in x, parts of
+// a bag in y (the kernels loop over what the grid leaves).
+struct BagGrid {
+  dim3 grid;
+  int32_t lg;
+};
+
+BagGrid bag_grid(int64_t bags, int64_t chunks_per_bag) {
+  const int64_t chunks = chunks_per_bag > 0 ? chunks_per_bag : 1;
+  BagGrid g;
+  g.lg = chunks <= 16 * kJagItems ? 4 : (chunks <= 64 * kJagItems ? 6 : 8);
+  int64_t parts = ceil_div(chunks, static_cast<int64_t>(kJagItems) << g.lg);
+  if (parts > 64) parts = 64;
+  int64_t x = ceil_div(bags, int64_t(1) << (8 - g.lg));
+  if (x > (int64_t(1) << 30)) x = int64_t(1) << 30;
+  g.grid = dim3(static_cast<uint32_t>(x), static_cast<uint32_t>(parts));
+  return g;
 }
 
 int pick_vec(int64_t row_bytes, std::initializer_list<const void*> ptrs) {
@@ -338,12 +327,6 @@ int pick_vec(int64_t row_bytes, std::initializer_list<const void*> ptrs) {
     if (ok) return vec;
   }
   return 1;
-}
-
-int grid_for(int64_t items) {
-  const int64_t blocks = ceil_div(items, 256);
-  const int64_t cap = static_cast<int64_t>(num_cus()) * 32;
-  return static_cast<int>(blocks < 1 ? 1 : (blocks > cap ? cap : blocks));
 }
 
 int build_meta(JaggedMeta& m, int32_t ndim, const void* const* offsets, int32_t offset_bytes,
@@ -421,25 +404,18 @@ extern "C" int mx_jagged_to_padded_dense(const void* values, int64_t elem_bytes,
   auto* s = as_stream(stream);
   const auto* v = static_cast<const uint8_t*>(values);
   auto* o = static_cast<uint8_t*>(out);
-  const int64_t nbags = offsets_numel[0] - 1;
-  const bool one = num_jagged_dim == 1 && nbags <= 0x7fffffffll;
-  const int grid = one ? 0 : grid_for(rows * vpr);  // the one-dim grid is per bag
+  const int64_t max_L = max_lengths[num_jagged_dim - 1];
+  const int64_t nbags = rows / max_L;  // rows > 0: max_L > 0
+  const BagGrid g = bag_grid(nbags, max_L * vpr);
+  const bool one = num_jagged_dim == 1 && g.lg == 8;
   MX_VEC_SWITCH(vec, {
     Chunk<V> pad;
     for (int i = 0; i < V; ++i) pad.b[i] = pat[i];
-    if (one) {
-      const dim3 g = grid_1d(nbags, max_lengths[0] * vpr);
-      if (offset_bytes == 8)
-        j2pd1_kernel<V, int64_t><<<g, 256, 0, s>>>(
-            v, o, static_cast<const int64_t*>(offsets[0]), max_lengths[0], vpr, pad);
-      else
-        j2pd1_kernel<V, int32_t><<<g, 256, 0, s>>>(
-            v, o, static_cast<const int32_t*>(offsets[0]), max_lengths[0], vpr, pad);
-    } else if (offset_bytes == 8) {
-      j2pd_kernel<V, int64_t><<<grid, 256, 0, s>>>(v, o, m, rows, vpr, pad);
-    } else {
-      j2pd_kernel<V, int32_t><<<grid, 256, 0, s>>>(v, o, m, rows, vpr, pad);
-    }
+    const auto kernel = one ? (offset_bytes == 8 ? j2pd_kernel<V, int64_t, true>
+                                                 : j2pd_kernel<V, int32_t, true>)
+                            : (offset_bytes == 8 ? j2pd_kernel<V, int64_t, false>
+                                                 : j2pd_kernel<V, int32_t, false>);
+    kernel<<<g.grid, 256, 0, s>>>(v, o, m, nbags, g.lg, vpr, pad);
   });
   MX_LAUNCH_CHECK();
   return MX_OK;
@@ -471,25 +447,18 @@ static int jagged_output_op(const void* dense, int64_t elem_bytes, int64_t inner
   auto* s = as_stream(stream);
   const auto* d = static_cast<const uint8_t*>(dense);
   auto* o = static_cast<uint8_t*>(out);
-  const int64_t nbags = offsets_numel[0] - 1;
-  const bool one = num_jagged_dim == 1 && nbags < 0x7fffffffll;
-  const int grid = one ? 0 : grid_for(total_L * vpr);  // the one-dim grid is per bag
-  const dim3 g1 = grid_1d(nbags + 1, max_lengths[0] * vpr);
-  const int64_t L0 = max_lengths[0];
+  const int last = num_jagged_dim - 1;
+  const int64_t nlists = offsets_numel[last] - 1;
+  const BagGrid g = bag_grid(nlists + 1, max_lengths[last] * vpr);
+  const bool one = num_jagged_dim == 1 && g.lg == 8;
   if (x_values == nullptr) {
     MX_VEC_SWITCH(vec, {
-      if (one) {
-        if (offset_bytes == 8)
-          jagged_out1_kernel<V, int64_t, false, MX_DTYPE_F32, false><<<g1, 256, 0, s>>>(
-              d, nullptr, o, static_cast<const int64_t*>(offsets[0]), nbags, L0, total_L, vpr);
-        else
-          jagged_out1_kernel<V, int32_t, false, MX_DTYPE_F32, false><<<g1, 256, 0, s>>>(
-              d, nullptr, o, static_cast<const int32_t*>(offsets[0]), nbags, L0, total_L, vpr);
-      } else if (offset_bytes == 8) {
-        d2j_kernel<V, int64_t><<<grid, 256, 0, s>>>(d, o, m, total_L, vpr);
-      } else {
-        d2j_kernel<V, int32_t><<<grid, 256, 0, s>>>(d, o, m, total_L, vpr);
-      }
+      constexpr int F = MX_DTYPE_F32;  // a copy: no element type
+      const auto kernel = one ? (offset_bytes == 8 ? jagged_out_kernel<V, int64_t, false, F, false, true>
+                                                   : jagged_out_kernel<V, int32_t, false, F, false, true>)
+                              : (offset_bytes == 8 ? jagged_out_kernel<V, int64_t, false, F, false, false>
+                                                   : jagged_out_kernel<V, int32_t, false, F, false, false>);
+      kernel<<<g.grid, 256, 0, s>>>(d, nullptr, o, m, nlists, g.lg, total_L, vpr);
     });
     MX_LAUNCH_CHECK();
     return MX_OK;
@@ -500,16 +469,12 @@ static int jagged_output_op(const void* dense, int64_t elem_bytes, int64_t inner
 #define MX_OP_LAUNCH(DTC, MULC)                                                                 \
   MX_VEC_SWITCH(vec, {                                                                          \
     if constexpr (V >= BinOp<DTC, MULC>::kBytes) {                                              \
-      if (one && offset_bytes == 8)                                                             \
-        jagged_out1_kernel<V, int64_t, true, DTC, MULC><<<g1, 256, 0, s>>>(                     \
-            d, x, o, static_cast<const int64_t*>(offsets[0]), nbags, L0, total_L, vpr);         \
-      else if (one)                                                                             \
-        jagged_out1_kernel<V, int32_t, true, DTC, MULC><<<g1, 256, 0, s>>>(                     \
-            d, x, o, static_cast<const int32_t*>(offsets[0]), nbags, L0, total_L, vpr);         \
-      else if (offset_bytes == 8)                                                               \
-        jagged_add_kernel<V, int64_t, DTC, MULC><<<grid, 256, 0, s>>>(x, d, o, m, total_L, vpr); \
-      else                                                                                      \
-        jagged_add_kernel<V, int32_t, DTC, MULC><<<grid, 256, 0, s>>>(x, d, o, m, total_L, vpr); \
+      const auto kernel =                                                                       \
+          one ? (offset_bytes == 8 ? jagged_out_kernel<V, int64_t, true, DTC, MULC, true>       \
+                                   : jagged_out_kernel<V, int32_t, true, DTC, MULC, true>)      \
+              : (offset_bytes == 8 ? jagged_out_kernel<V, int64_t, true, DTC, MULC, false>      \
+                                   : jagged_out_kernel<V, int32_t, true, DTC, MULC, false>);    \
+      kernel<<<g.grid, 256, 0, s>>>(d, x, o, m, nlists, g.lg, total_L, vpr);                    \
     }                                                                                           \
   })
 #define MX_ADD_LAUNCH(DTC)    \
