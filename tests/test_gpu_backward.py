@@ -249,6 +249,36 @@ def _backward_case(dev, inp, pooling, wd=0.0, wd_mode=0, lr=0.01, eps=1e-8, seed
     return Wg, W_exp
 
 
+@pytest.mark.parametrize("N", [1, 63, 64, 65, 1023, 1024, 1025, 2048, 2049, 4096, 4097, 8191, 8192,
+                               8193])
+@pytest.mark.parametrize("E,B", [(1, 7), (40, 3000), (70000, 50), ((1 << 24) + 1, 300)])
+def test_small_batch_edges(dev, N, E, B):
+    """Batches up to 8192 positions take the one-block transpose, one more the
+    chain of launches: the layout bit-exact at every count of keys per lane and
+    of digit passes, with one run, long runs, and more bags than positions;
+    the update against the oracle, weighted and not."""
+    print(f"[case] small batch N={N} E={E} B={B}", flush=True)
+    rng = np.random.default_rng(N + E)
+    inp = _bag_input(rng, E, rng.integers(0, E, size=N), B)
+    _check_transpose(dev, inp)
+    _check_transpose(dev, inp, torch.int32)
+    # Long runs sum in chunks, the oracle in sequence: compared where runs are short.
+    if E >= 70000 and E < 1 << 24:
+        _backward_case(dev, inp, 0, seed=3, weighted=N % 2 == 0)
+
+
+@pytest.mark.parametrize("weighted", [False, True])
+def test_small_batch_backward(dev, weighted):
+    """The one-block transpose's chunk layout: runs of 24 to a few hundred
+    occurrences, over features with and without a table of their own."""
+    print(f"[case] small batch backward weighted={weighted}", flush=True)
+    rng = np.random.default_rng(77 + weighted)
+    inp = random_tbe(rng, 3, 100, [64, 64, 64], [60, 9, 30000], 30)
+    assert inp.N <= 8192
+    _backward_case(dev, inp, 0, seed=5, weighted=weighted)
+    _backward_case(dev, inp, 1, seed=6, weighted=weighted, index_dtype=torch.int32)
+
+
 @pytest.mark.parametrize("pooling", [0, 1])
 @pytest.mark.parametrize("T,B,dims,rows,max_L,dup", [
     (2, 40, [128, 128], [300, 300], 20, False),
