@@ -25,6 +25,8 @@
 // block ranks its bags by length and gives bags of similar length to one
 // wave (config 2: 36.7 -> 35.9 us cold, 34.1 -> 33.3 us over rotating
 // batches).
+#include <type_traits>
+
 #include "mx_common.h"
 
 namespace mx {
@@ -192,11 +194,95 @@ constexpr int fwd_waves() {
   return (NCH == 1 && !WEIGHTED && sizeof(I) == 8) ? 8 : 1;
 }
 
+// One bag of one group: its rows summed in index order and stored.
+template <typename I, typename WT, int G, int NCH, int U, bool WEIGHTED, bool OUT_F16>
+__device__ __forceinline__ void pool_bag(const WT* __restrict__ Wt, __amdgpu_buffer_rsrc_t rsrc,
+                                         bool one_table, int32_t D,
+                                         const I* __restrict__ indices,
+                                         const float* __restrict__ iw, int64_t start, int64_t end,
+                                         int32_t pooling, void* __restrict__ out, int64_t obase,
+                                         int g, int k) {
+  float acc[NCH][4];
+#pragma unroll
+  for (int c = 0; c < NCH; ++c)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[c][e] = 0.0f;
+  bool active[NCH];
+  const WT* lane_col[NCH];   // this lane's first column of each chunk, row 0
+  uint32_t lane_byte[NCH];   // the same as a byte offset in the table
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    active[c] = (c * G + k) * 4 < D;
+    // A chunk past the row's end reads the row's first columns instead (never
+    // stored), so that no load sits behind a branch.
+    const int col = active[c] ? (c * G + k) * 4 : 0;
+    lane_col[c] = Wt + col;
+    lane_byte[c] = static_cast<uint32_t>(col * sizeof(WT));
+  }
+
+  // The group's indices come G at a time, one batch ahead of its rows, so a
+  // bag longer than G does not wait for its next batch of indices.
+  I nxt_idx = start + k < end ? indices[start + k] : I(0);
+  float nxt_w = 0.0f;
+  if constexpr (WEIGHTED) nxt_w = start + k < end ? iw[start + k] : 0.0f;
+  for (int64_t base = start; base < end; base += G) {
+    const int n = static_cast<int>(end - base < G ? end - base : G);
+    const I cur_idx = nxt_idx;
+    [[maybe_unused]] const float my_w = nxt_w;
+    if (base + G + k < end) {
+      nxt_idx = indices[base + G + k];
+      if constexpr (WEIGHTED) nxt_w = iw[base + G + k];
+    }
+    // The lane that loads an index also turns it into the row's offset,
+    // once, instead of every lane of the group per row: in bytes for buffer
+    // loads when every row of the batch ends below 4 GiB into its table (one
+    // 32-bit word per row between lanes, one 32-bit add per load), else in
+    // elements for 64-bit addresses.
+    const uint64_t my_elem = k < n ? static_cast<uint64_t>(cur_idx) * static_cast<uint64_t>(D) : 0;
+    const uint64_t my_end = (my_elem + static_cast<uint64_t>(D)) * sizeof(WT);
+    if (one_table && __all(my_end <= 0xffffffffull))  // wave-uniform
+      pool_batch<true, WT, G, NCH, U, WEIGHTED>(my_elem * sizeof(WT), my_w, n, g, lane_col, rsrc,
+                                               lane_byte, acc);
+    else  // a wave over two tables, or a table past 4 GiB: half the rows in flight
+      pool_batch<false, WT, G, NCH, (U > 1 ? U / 2 : 1), WEIGHTED>(my_elem, my_w, n, g, lane_col,
+                                                                 rsrc, lane_byte, acc);
+  }
+  const int64_t L = end - start;
+  if (pooling == MX_POOL_MEAN && L > 0) {
+    const float inv = 1.0f / static_cast<float>(L);
+#pragma unroll
+    for (int c = 0; c < NCH; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[c][e] *= inv;
+  }
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    if (!active[c]) continue;
+    const int64_t col = obase + (c * G + k) * 4;
+    if constexpr (OUT_F16) {
+      __half* o = reinterpret_cast<__half*>(out) + col;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = __float2half_rn(acc[c][e]);
+    } else {
+      *reinterpret_cast<float4*>(reinterpret_cast<float*>(out) + col) =
+          make_float4(acc[c][0], acc[c][1], acc[c][2], acc[c][3]);
+    }
+  }
+}
+
+// Rows in flight per lane of NCH chunks.
+template <int NCH>
+constexpr int fwd_rows() {
+  return NCH <= 1 ? 8 : (NCH <= 2 ? 4 : 2);
+}
+
 // A wave serves 64/G bags at once, G lanes per bag, lane k owning columns
 // (c*G + k)*4 .. +4 (float4 loads: a D=128 row is one 512 B access of 32
 // lanes).  Several bags per wave keep several independent offsets -> indices
 // -> rows chains in flight; each column is still summed in index order.
-template <typename I, typename WT, int G, int NCH, int U, bool WEIGHTED, bool OUT_F16>
+// MIXED: tables of different widths; G fits the narrow ones and a wave takes
+// 1, 2 or NCH chunks per lane by its bags' own widths.
+template <typename I, typename WT, int G, int NCH, bool MIXED, bool WEIGHTED, bool OUT_F16>
 __global__ void __launch_bounds__(256)
     __attribute__((amdgpu_waves_per_eu(fwd_waves<I, NCH, WEIGHTED>())))
     tbe_fwd_group_kernel(const WT* __restrict__ W, const int64_t* __restrict__ w_off,
@@ -265,82 +351,121 @@ __global__ void __launch_bounds__(256)
   const bool one_table = __all(t == tw);  // wave-uniform
   const __amdgpu_buffer_rsrc_t rsrc = table_rsrc(W + w_off[tw]);
 
-  float acc[NCH][4];
-#pragma unroll
-  for (int c = 0; c < NCH; ++c)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) acc[c][e] = 0.0f;
-  bool active[NCH];
-  const WT* lane_col[NCH];   // this lane's first column of each chunk, row 0
-  uint32_t lane_byte[NCH];   // the same as a byte offset in the table
-#pragma unroll
-  for (int c = 0; c < NCH; ++c) {
-    active[c] = (c * G + k) * 4 < D;
-    // A chunk past the row's end reads the row's first columns instead (never
-    // stored), so that no load sits behind a branch.
-    const int col = active[c] ? (c * G + k) * 4 : 0;
-    lane_col[c] = Wt + col;
-    lane_byte[c] = static_cast<uint32_t>(col * sizeof(WT));
-  }
-
-  // The group's indices come G at a time, one batch ahead of its rows, so a
-  // bag longer than G does not wait for its next batch of indices.
-  I nxt_idx = start + k < end ? indices[start + k] : I(0);
-  float nxt_w = 0.0f;
-  if constexpr (WEIGHTED) nxt_w = start + k < end ? iw[start + k] : 0.0f;
-  for (int64_t base = start; base < end; base += G) {
-    const int n = static_cast<int>(end - base < G ? end - base : G);
-    const I cur_idx = nxt_idx;
-    [[maybe_unused]] const float my_w = nxt_w;
-    if (base + G + k < end) {
-      nxt_idx = indices[base + G + k];
-      if constexpr (WEIGHTED) nxt_w = iw[base + G + k];
-    }
-    // The lane that loads an index also turns it into the row's offset,
-    // once, instead of every lane of the group per row: in bytes for buffer
-    // loads when every row of the batch ends below 4 GiB into its table (one
-    // 32-bit word per row between lanes, one 32-bit add per load), else in
-    // elements for 64-bit addresses.
-    const uint64_t my_elem = k < n ? static_cast<uint64_t>(cur_idx) * static_cast<uint64_t>(D) : 0;
-    const uint64_t my_end = (my_elem + static_cast<uint64_t>(D)) * sizeof(WT);
-    if (one_table && __all(my_end <= 0xffffffffull))  // wave-uniform
-      pool_batch<true, WT, G, NCH, U, WEIGHTED>(my_elem * sizeof(WT), my_w, n, g, lane_col, rsrc,
-                                               lane_byte, acc);
-    else  // a wave over two tables, or a table past 4 GiB: half the rows in flight
-      pool_batch<false, WT, G, NCH, (U > 1 ? U / 2 : 1), WEIGHTED>(my_elem, my_w, n, g, lane_col,
-                                                                 rsrc, lane_byte, acc);
-  }
-  const int64_t L = end - start;
-  if (pooling == MX_POOL_MEAN && L > 0) {
-    const float inv = 1.0f / static_cast<float>(L);
-#pragma unroll
-    for (int c = 0; c < NCH; ++c)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) acc[c][e] *= inv;
-  }
   const int64_t obase = bm.out_base(bag, b, D0);
-#pragma unroll
-  for (int c = 0; c < NCH; ++c) {
-    if (!active[c]) continue;
-    const int64_t col = obase + (c * G + k) * 4;
-    if constexpr (OUT_F16) {
-      __half* o = reinterpret_cast<__half*>(out) + col;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) o[e] = __float2half_rn(acc[c][e]);
-    } else {
-      *reinterpret_cast<float4*>(reinterpret_cast<float*>(out) + col) =
-          make_float4(acc[c][0], acc[c][1], acc[c][2], acc[c][3]);
-    }
+#define MX_POOL(N)                                                                              \
+  pool_bag<I, WT, G, N, fwd_rows<N>(), WEIGHTED, OUT_F16>(Wt, rsrc, one_table, D, indices, iw, \
+                                                          start, end, pooling, out, obase, g, k)
+  if constexpr (MIXED) {
+    if (__all(D <= 4 * G))  // wave-uniform
+      MX_POOL(1);
+    else if (__all(D <= 8 * G))
+      MX_POOL(2);
+    else
+      MX_POOL(NCH);
+  } else {
+    MX_POOL(NCH);
   }
+#undef MX_POOL
 }
 
 // Gradient of the per-sample weights of a weighted lookup:
 //   grad_iw[l] = sum_d grad_output[b, D_off[t] + d] * W_t[idx[l], d]
 // (MEAN: times 1/L), 0 for tables whose feature_requires_grad entry is 0.
-// Same G-lane-per-bag mapping as the forward; the bag's gradient slice stays
-// in registers, each row's dot product is reduced over the group in a fixed
-// xor-tree order.
+// Same G-lane-per-bag mapping as the forward (and its buffer loads and index
+// prefetch); the bag's gradient slice stays in registers.  The U rows in flight
+// reduce together: each step halves the rows a lane holds while it adds the
+// other half of the group, so U rows take U - 1 + log2(G / U) exchanges instead
+// of U * log2(G), and lane r * G/U ends with row r's dot product (a fixed tree).
+// (20 fp16 tables of six widths up to 256, 295k lookups: 50.5 us with branches
+// around the loads and a tree per row, 21.1.)
+template <int G, int U>
+__device__ __forceinline__ float reduce_rows(float (&d)[U], int k) {
+#pragma unroll
+  for (int s = U / 2, m = G / 2; s >= 1; s >>= 1, m >>= 1) {
+    const bool up = (k & m) != 0;
+#pragma unroll
+    for (int i = 0; i < s; ++i) {
+      const float send = up ? d[i] : d[i + s];
+      const float keep = up ? d[i + s] : d[i];
+      d[i] = keep + __shfl_xor(send, m, 64);
+    }
+  }
+#pragma unroll
+  for (int m = G / U / 2; m >= 1; m >>= 1) d[0] += __shfl_xor(d[0], m, 64);
+  return d[0];
+}
+
 template <typename I, typename WT, int G, int NCH, int U>
+__device__ __forceinline__ void dot_bag(const float* __restrict__ grad_row,
+                                        const WT* __restrict__ Wt, __amdgpu_buffer_rsrc_t rsrc,
+                                        bool one_table, int32_t D, const I* __restrict__ indices,
+                                        int64_t start, int64_t end, int32_t pooling,
+                                        float* __restrict__ out, int g, int k) {
+  float gv[NCH][4];
+  bool active[NCH];
+  const WT* lane_col[NCH];
+  uint32_t lane_byte[NCH];
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    active[c] = (c * G + k) * 4 < D;
+    // A chunk past the row's end reads the row's first columns (left out of the
+    // sum, also where they are not finite), so that no load sits behind a branch.
+    const int col = active[c] ? (c * G + k) * 4 : 0;
+    lane_col[c] = Wt + col;
+    lane_byte[c] = static_cast<uint32_t>(col * sizeof(WT));
+    load_vec<4>(grad_row + col, gv[c]);
+  }
+  const int64_t L = end - start;
+  const float inv = (pooling == MX_POOL_MEAN && L > 0) ? 1.0f / static_cast<float>(L) : 1.0f;
+  I nxt_idx = start + k < end ? indices[start + k] : I(0);
+  for (int64_t base = start; base < end; base += G) {
+    const int n = static_cast<int>(end - base < G ? end - base : G);
+    const I cur_idx = nxt_idx;
+    if (base + G + k < end) nxt_idx = indices[base + G + k];
+    const uint64_t my_elem = k < n ? static_cast<uint64_t>(cur_idx) * static_cast<uint64_t>(D) : 0;
+    const uint64_t my_end = (my_elem + static_cast<uint64_t>(D)) * sizeof(WT);
+    auto rows = [&](auto buf) {
+      for (int j = 0; j < n; j += U) {
+        float v[U][NCH][4];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int r = j + u < n ? j + u : n - 1;
+          if constexpr (decltype(buf)::value) {
+            const uint32_t off = __shfl(static_cast<uint32_t>(my_elem * sizeof(WT)), g * G + r, 64);
+#pragma unroll
+            for (int c = 0; c < NCH; ++c) buf_row4(rsrc, off + lane_byte[c], lane_col[c], v[u][c]);
+          } else {
+            const uint64_t off = __shfl(my_elem, g * G + r, 64);
+#pragma unroll
+            for (int c = 0; c < NCH; ++c) load_row4(lane_col[c] + off, v[u][c]);
+          }
+        }
+        float dot[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          dot[u] = 0.0f;
+#pragma unroll
+          for (int c = 0; c < NCH; ++c) {
+            float x = dot[u];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x = __builtin_fmaf(gv[c][e], v[u][c][e], x);
+            dot[u] = active[c] ? x : dot[u];
+          }
+        }
+        const float sum = reduce_rows<G, U>(dot, k);
+        const int r = k / (G / U);
+        if (k % (G / U) == 0 && j + r < n)
+          out[base + j + r] = pooling == MX_POOL_MEAN ? __fmul_rn(sum, inv) : sum;
+      }
+    };
+    if (one_table && __all(my_end <= 0xffffffffull))  // wave-uniform
+      rows(std::true_type{});
+    else
+      rows(std::false_type{});
+  }
+}
+
+template <typename I, typename WT, int G, int NCH, bool MIXED>
 __global__ void __launch_bounds__(256)
     grad_indice_weights_kernel(const float* __restrict__ grad, BagMap bm,
                                const WT* __restrict__ W, const int64_t* __restrict__ w_off,
@@ -364,79 +489,75 @@ __global__ void __launch_bounds__(256)
   }
   const int32_t D0 = D_off[t];
   const int32_t D = D_off[t + 1] - D0;
-  const WT* __restrict__ Wt = W + w_off[t];
-  bool active[NCH];
-  float gv[NCH][4];
-#pragma unroll
-  for (int c = 0; c < NCH; ++c) {
-    active[c] = (c * G + k) * 4 < D;
-    if (active[c])
-      load_vec<4>(grad + bm.out_base(bag, b, D0) + (c * G + k) * 4, gv[c]);
+  if (D <= 0) {  // no columns: every dot product is empty
+    for (int64_t l = start + k; l < end; l += G) out[l] = 0.0f;
+    return;
+  }
+  const int64_t tw = readlane_i64(t, __builtin_amdgcn_readfirstlane(lane));
+  const bool one_table = __all(t == tw);  // wave-uniform
+  const __amdgpu_buffer_rsrc_t rsrc = table_rsrc(W + w_off[tw]);
+  const float* grad_row = grad + bm.out_base(bag, b, D0);
+#define MX_DOT(N)                                                                                \
+  dot_bag<I, WT, G, N, fwd_rows<N>()>(grad_row, W + w_off[t], rsrc, one_table, D, indices, start, \
+                                      end, pooling, out, g, k)
+  if constexpr (MIXED) {
+    if (__all(D <= 4 * G))  // wave-uniform
+      MX_DOT(1);
+    else if (__all(D <= 8 * G))
+      MX_DOT(2);
     else
-      gv[c][0] = gv[c][1] = gv[c][2] = gv[c][3] = 0.0f;
+      MX_DOT(NCH);
+  } else {
+    MX_DOT(NCH);
   }
-  const int64_t L = end - start;
-  const float inv = (pooling == MX_POOL_MEAN && L > 0) ? 1.0f / static_cast<float>(L) : 1.0f;
-  for (int64_t base = start; base < end; base += G) {
-    const int n = static_cast<int>(end - base < G ? end - base : G);
-    const int64_t my_idx = k < n ? static_cast<int64_t>(indices[base + k]) : 0;
-    for (int j = 0; j < n; j += U) {
-      float v[U][NCH][4];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if (j + u < n) {
-          const int64_t r = __shfl(my_idx, g * G + j + u, 64);
-#pragma unroll
-          for (int c = 0; c < NCH; ++c)
-            if (active[c]) load_row4(Wt + r * D + (c * G + k) * 4, v[u][c]);
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if (j + u < n) {
-          float dot = 0.0f;
-#pragma unroll
-          for (int c = 0; c < NCH; ++c)
-            if (active[c])
-#pragma unroll
-              for (int e = 0; e < 4; ++e) dot = __builtin_fmaf(gv[c][e], v[u][c][e], dot);
-#pragma unroll
-          for (int m = G / 2; m >= 1; m >>= 1) dot += __shfl_xor(dot, m, 64);
-          if (k == 0) out[base + j + u] = pooling == MX_POOL_MEAN ? __fmul_rn(dot, inv) : dot;
-        }
-      }
-    }
-  }
+#undef MX_DOT
 }
 
-template <typename I, typename WT, int G, int NCH, bool WEIGHTED, bool OUT_F16>
+// Tables of different widths (a fixed batch says so: total_D) whose mean is at
+// most three quarters of the widest: there the lanes that fit the widest rows
+// are half idle or more (six widths up to 256: forward 22.6 -> 20.9 us, 512, 64
+// and 32 a training step 201 -> 182).  Nearer the widest, more lanes per bag
+// keep more rows in flight.
+bool mixed_widths(const BagMap& bm, int32_t T, int32_t max_D) {
+  return bm.total_D > 0 && max_D > 64 && 4 * bm.total_D <= 3ll * T * max_D;
+}
+
+template <typename I, typename WT, int G, int NCH, bool MIXED, bool WEIGHTED, bool OUT_F16>
 void launch_fwd_group(hipStream_t s, const WT* W, const int64_t* w_off, const int32_t* D_off,
                       const BagMap& bm, const void* idx, const void* off, int32_t pooling,
                       const float* iw, void* out, int64_t nbags) {
-  constexpr int U = NCH <= 1 ? 8 : (NCH <= 2 ? 4 : 2);  // rows in flight per lane
   constexpr int P = 64 / G;
   const int64_t grid = ceil_div(nbags, kWavesPerBlock * P);
-  tbe_fwd_group_kernel<I, WT, G, NCH, U, WEIGHTED, OUT_F16><<<dim3(static_cast<uint32_t>(grid)), 256, 0, s>>>(
-      W, w_off, D_off, bm, static_cast<const I*>(idx), static_cast<const I*>(off), pooling, iw, out,
-      nbags);
+  tbe_fwd_group_kernel<I, WT, G, NCH, MIXED, WEIGHTED, OUT_F16>
+      <<<dim3(static_cast<uint32_t>(grid)), 256, 0, s>>>(
+          W, w_off, D_off, bm, static_cast<const I*>(idx), static_cast<const I*>(off), pooling, iw,
+          out, nbags);
 }
 
 template <typename I, typename WT, bool WEIGHTED, bool OUT_F16>
-int dispatch_fwd(hipStream_t s, int32_t max_D, const WT* W, const int64_t* w_off,
+int dispatch_fwd(hipStream_t s, int32_t T, int32_t max_D, const WT* W, const int64_t* w_off,
                  const int32_t* D_off, const BagMap& bm, const void* idx, const void* off,
                  int32_t pooling, const float* iw, void* out, int64_t nbags) {
-#define MX_FWD_G(G, NCH) \
-  launch_fwd_group<I, WT, G, NCH, WEIGHTED, OUT_F16>(s, W, w_off, D_off, bm, idx, off, pooling, iw, out, nbags)
+#define MX_FWD_G(G, NCH, MIXED) \
+  launch_fwd_group<I, WT, G, NCH, MIXED, WEIGHTED, OUT_F16>(s, W, w_off, D_off, bm, idx, off, \
+                                                            pooling, iw, out, nbags)
+  const bool mixed = mixed_widths(bm, T, max_D);
   if (max_D <= 64)
-    MX_FWD_G(16, 1);  // 4 bags per wave
+    MX_FWD_G(16, 1, false);  // 4 bags per wave
+  else if (mixed && max_D <= 256)
+    MX_FWD_G(16, 4, true);
+  else if (mixed && max_D <= 512)
+    MX_FWD_G(32, 4, true);
   else if (max_D <= 128)
-    MX_FWD_G(32, 1);  // 2 bags per wave, one D=128 row per 32 lanes x 16 B
+    MX_FWD_G(32, 1, false);  // 2 bags per wave, one D=128 row per 32 lanes x 16 B
   else if (max_D <= 256)
-    MX_FWD_G(64, 1);
+    MX_FWD_G(64, 1, false);
   else if (max_D <= 512)
-    MX_FWD_G(64, 2);
+    MX_FWD_G(64, 2, false);
+  else if (mixed)
+    MX_FWD_G(64, 4, true);
   else
-    MX_FWD_G(64, 4);
+    MX_FWD_G(64, 4, false);
 #undef MX_FWD_G
   return MX_OK;
 }
@@ -593,7 +714,7 @@ int tbe_forward_impl(const void* weights, int32_t weights_ty, const int64_t* wei
   auto* s = as_stream(stream);
   const bool w = indice_weights != nullptr;
   const bool h = out_dtype == MX_SPARSE_FP16;
-#define MX_ARGS(WT) s, max_D, static_cast<const WT*>(weights), weights_offsets, D_offsets, bm, \
+#define MX_ARGS(WT) s, T, max_D, static_cast<const WT*>(weights), weights_offsets, D_offsets, bm, \
                 indices, offsets, pooling_mode, indice_weights, out, nbags
 #define MX_FWD_W(I, WT)                                                                          \
   if (w)                                                                                         \
@@ -716,15 +837,16 @@ int grad_indice_weights_impl(const float* grad_output, const BagMap& bm, const v
                  grad_indice_weights,
              "null pointer argument");
   auto* s = as_stream(stream);
-#define MX_GIW(I, G, NCH, U)                                                                   \
+  const bool mixed = mixed_widths(bm, T, max_D);
+#define MX_GIW(I, G, NCH, MIXED)                                                               \
   do {                                                                                         \
     if (weights_ty == MX_SPARSE_FP16)                                                          \
-      MX_GIW_T(I, __half, G, NCH, U);                                                          \
+      MX_GIW_T(I, __half, G, NCH, MIXED);                                                      \
     else                                                                                       \
-      MX_GIW_T(I, float, G, NCH, U);                                                           \
+      MX_GIW_T(I, float, G, NCH, MIXED);                                                       \
   } while (0)
-#define MX_GIW_T(I, WT, G, NCH, U)                                                             \
-  grad_indice_weights_kernel<I, WT, G, NCH, U><<<dim3(static_cast<uint32_t>(                  \
+#define MX_GIW_T(I, WT, G, NCH, MIXED)                                                         \
+  grad_indice_weights_kernel<I, WT, G, NCH, MIXED><<<dim3(static_cast<uint32_t>(              \
                                                ceil_div(nbags, kWavesPerBlock * (64 / G)))),   \
                                            256, 0, s>>>(                                      \
       grad_output, bm, static_cast<const WT*>(weights), weights_offsets, D_offsets,            \
@@ -732,15 +854,21 @@ int grad_indice_weights_impl(const float* grad_output, const BagMap& bm, const v
       feature_requires_grad, grad_indice_weights, nbags)
 #define MX_GIW_D(I)                 \
   if (max_D <= 64)                  \
-    MX_GIW(I, 16, 1, 8);            \
+    MX_GIW(I, 16, 1, false);        \
+  else if (mixed && max_D <= 256)   \
+    MX_GIW(I, 16, 4, true);         \
+  else if (mixed && max_D <= 512)   \
+    MX_GIW(I, 32, 4, true);         \
   else if (max_D <= 128)            \
-    MX_GIW(I, 32, 1, 8);            \
+    MX_GIW(I, 32, 1, false);        \
   else if (max_D <= 256)            \
-    MX_GIW(I, 64, 1, 8);            \
+    MX_GIW(I, 64, 1, false);        \
   else if (max_D <= 512)            \
-    MX_GIW(I, 64, 2, 4);            \
+    MX_GIW(I, 64, 2, false);        \
+  else if (mixed)                   \
+    MX_GIW(I, 64, 4, true);         \
   else                              \
-    MX_GIW(I, 64, 4, 2);
+    MX_GIW(I, 64, 4, false);
   if (index_bytes == 8) {
     MX_GIW_D(int64_t)
   } else {
