@@ -514,12 +514,12 @@ __global__ void __launch_bounds__(256)
 }
 
 // Tables of different widths (a fixed batch says so: total_D) whose mean is at
-// most three quarters of the widest: there the lanes that fit the widest rows
-// are half idle or more (six widths up to 256: forward 22.6 -> 20.9 us, 512, 64
-// and 32 a training step 201 -> 182).  Nearer the widest, more lanes per bag
-// keep more rows in flight.
+// most five eighths of the widest: there the lanes that fit the widest rows
+// are half idle or more (six widths from 32 to 256: 22.6 -> 20.9 us).  Nearer the
+// widest, more lanes per bag keep more rows in flight (128 and 64 in turn: a
+// training step 137.0 us, 138.5 mixed).
 bool mixed_widths(const BagMap& bm, int32_t T, int32_t max_D) {
-  return bm.total_D > 0 && max_D > 64 && 4 * bm.total_D <= 3ll * T * max_D;
+  return bm.total_D > 0 && max_D > 64 && 8 * bm.total_D <= 5ll * T * max_D;
 }
 
 template <typename I, typename WT, int G, int NCH, bool MIXED, bool WEIGHTED, bool OUT_F16>
