@@ -243,11 +243,11 @@ int run_bounds(const int64_t* rows, void* indices, void* offsets, int64_t nbags,
                const int32_t* B_offsets, int32_t T, int64_t N, int32_t mode,
                unsigned long long* warning, const BoundsWs& w, hipStream_t s) {
   // Bags per block: between 32 and 256, the most that leaves eight blocks per
-  // CU, or fewer where their positions pass one round of loads.
+  // CU or about 512 positions per block (fewer, longer blocks cost a small batch
+  // its latency, shorter ones are mostly their own scan).
   int32_t bpb = kMaxBagsPerBlock;
-  const int64_t round = 256 * kIdxPerThread * static_cast<int64_t>(16 / sizeof(I));
   const int64_t fill = static_cast<int64_t>(num_cus()) * 8;
-  while (bpb > 32 && bpb * N > round * nbags && ceil_div(nbags, bpb) < fill) bpb >>= 1;
+  while (bpb > 32 && bpb * N > 512 * nbags && ceil_div(nbags, bpb) < fill) bpb >>= 1;
   if (w.ntiles > 1) {  // one tile: the blocks read their offsets themselves
     tile_max_kernel<I><<<dim3(static_cast<uint32_t>(ceil_div(w.ntiles, 4))), 256, 0, s>>>(
         static_cast<const I*>(offsets), nbags, N, w.tile, w.ntiles, w.tilemax);
