@@ -33,7 +33,7 @@
 //    keys and offsets.
 //  * Each run (one distinct (t, i)) is reduced by one G-lane group, lanes
 //    owning columns, occurrences added in sorted order.  Runs longer than
-//    kLong are cut into kChunk-occurrence chunks reduced in parallel into a
+//    long_run() are cut into kChunk-occurrence chunks reduced in parallel into a
 //    workspace, then summed in chunk order.  No atomics on data: results are
 //    deterministic.  Runs and chunks are split into one contiguous key range
 //    per XCD, so an XCD re-reads only its tables' gradient columns, from its
@@ -81,17 +81,26 @@ constexpr int kLinItems = 4;
 constexpr int kSegMaxT = 63;
 constexpr int64_t kSegRow = static_cast<int64_t>(kHistCopies) * kMaxPasses * kRadix;  // per feature
 constexpr int64_t kLinTile = 256 * kLinItems;         // positions per linearize block
-// Runs longer than kLong are chunked.  A wave's four short runs last as long
-// as the longest (two occurrences per round): 24 instead of 32 moves the
+// Runs longer than long_run() are chunked.  A wave's four short runs last as
+// long as the longest (two occurrences per round): 24 instead of 32 moves the
 // 13-16-round runs to the chunk path (config 3: 161.1 -> 158.8 us; 12, 16 and
-// 20 were within 1 us of it, 8 slower).
-constexpr int kLong = 24;
+// 20 were within 1 us of it, 8 slower).  Where the update's rows cost more per
+// occurrence -- wide ones, or widths the lanes do not divide -- 16 is better
+// (96-column sequences 150.5 -> 146.6 us, tables of 256, 200 and 168 columns
+// 201.6 -> 197.4, 256 123.4 -> 121.5), at full width up to 128 columns 24 stays
+// (64 columns: 152.6, 156.5 with 16; config 3: 201.3, 202.5).
+constexpr int kLongNarrow = 24;
+constexpr int kLongMin = 16;
+int32_t long_run(int32_t T, int32_t max_D, int64_t total_D) {
+  const bool full = total_D == static_cast<int64_t>(T) * max_D;
+  return full && (max_D == 64 || max_D == 128) ? kLongNarrow : kLongMin;
+}
 constexpr int kChunk = 32;                            // occurrences per chunk
 // One-pass scans per backward: run heads, chunk layout.
 constexpr int kScanSlots = 2;
-// Upper bound of the chunk count: sum over runs longer than kLong of
+// Upper bound of the chunk count: sum over runs longer than kLongMin of
 // ceil(len / kChunk) <= N / kChunk + (number of such runs).
-int64_t max_chunks(int64_t N) { return N / kChunk + N / (kLong + 1) + 2; }
+int64_t max_chunks(int64_t N) { return N / kChunk + N / (kLongMin + 1) + 2; }
 
 __device__ __forceinline__ uint32_t digit_mask(int bits, int p) {
   const int nb = bits - p * kRadixBits;
@@ -803,9 +812,10 @@ __global__ void __launch_bounds__(256)
 
 struct ChunkCount {
   const int32_t* cum;
+  int32_t long_len;
   __device__ uint32_t operator()(int64_t r) const {
     const int32_t len = cum[r + 1] - cum[r];
-    return len > kLong ? static_cast<uint32_t>((len + kChunk - 1) / kChunk) : 0u;
+    return len > long_len ? static_cast<uint32_t>((len + kChunk - 1) / kChunk) : 0u;
   }
 };
 
@@ -817,7 +827,7 @@ constexpr int kMarkEvery = 16;
 constexpr uint32_t kRunStart = 0x80000000u;
 
 // Epilogue of the chunk-count scan: chunk_start[r] = first chunk of run r
-// (runs of at most kLong occurrences own no chunk) and the chunk marks.
+// (runs of at most long_run() occurrences own no chunk) and the chunk marks.
 struct ChunkEpi {
   const int32_t* cum;
   uint32_t* chunk_start;
@@ -874,6 +884,7 @@ struct SmallSort {
   uint32_t* chunk_mark;
   uint32_t* total_chunks;
   int32_t max_chunks;     // entries of chunk_mark
+  uint32_t long_len;      // runs longer than this are chunked
 };
 
 // Sum over the block's waves before this one, and over all; a barrier on entry
@@ -1081,7 +1092,7 @@ __global__ void __launch_bounds__(kSweepThreads) small_transpose_kernel(SmallSor
       a.run_lengths[r] = static_cast<int32_t>(len);
       if (r >= runs) a.cum[r + 1] = N;
     }
-    if (len > static_cast<uint32_t>(kLong)) nq[it] = (len + kChunk - 1) / kChunk;
+    if (len > a.long_len) nq[it] = (len + kChunk - 1) / kChunk;
     own += nq[it];
   }
   if (!a.chunk_start) return;  // block-uniform
@@ -1254,6 +1265,7 @@ struct TransposeOut {
   int32_t* cum;         // [N+1]
   float* weights_sorted;  // [N] per-sample weights in sorted order, or null
   uint32_t* chunk_start;  // [N] long runs' chunks of a small batch (backward), or null
+  int32_t long_len;       // with chunk_start: runs longer than this are chunked
 };
 
 // Early words kept zero between calls.  Clearing a call's early words in its
@@ -1325,7 +1337,7 @@ int run_transpose(const int64_t* hsc, int32_t T, int64_t B, int64_t nbags,
                       o.linear, iw, w.vals[0], o.sorted, reinterpret_cast<uint32_t*>(o.infos),
                       o.weights_sorted, o.run, o.cum, o.run_lengths, o.num_runs, &w.counters[0],
                       w.fail, o.chunk_start, chunks ? w.chunk_mark : nullptr, &w.counters[1],
-                      static_cast<int32_t>(max_chunks(N))};
+                      static_cast<int32_t>(max_chunks(N)), static_cast<uint32_t>(o.long_len)};
     return index_bytes == 8 ? launch_small_transpose<int64_t>(a, s)
                             : launch_small_transpose<int32_t>(a, s);
   }
@@ -1446,6 +1458,7 @@ struct BwdArgs {
   int32_t nb;
   int32_t pooling;
   int32_t wd_mode;
+  int32_t long_len;  // runs longer than this are chunked
   float lr;
   float eps;
   float wd;
@@ -1868,7 +1881,7 @@ __global__ void __launch_bounds__(256) bwd_chunk_kernel(BwdArgs a) {
   }
 }
 
-// Pass B (runs of at most kLong occurrences): one G-lane group per run --
+// Pass B (runs of at most long_run() occurrences): one G-lane group per run --
 // gradient sum in sorted order, rowwise Adagrad, in-place update.  The
 // table of a run comes from the first batch of infos, which is kept for the
 // gradient sum.
@@ -1883,7 +1896,7 @@ __device__ __forceinline__ void short_run_body(const BwdArgs& a, const MetaView&
     const int64_t cs0 = a.cum[r];
     const int64_t cs1 = a.cum[r + 1];
     const int64_t ckey = a.run[r];
-    if (cs1 - cs0 > kLong) continue;  // long runs: long_run_body
+    if (cs1 - cs0 > a.long_len) continue;  // long runs: long_run_body
     const int32_t info0 = k < cs1 - cs0 ? a.infos[cs0 + k] : 0;
     const int64_t t = table_of(a, __shfl(info0, g * G, 64));
     const int32_t D = FULL ? G * NCH * 4 : mv.D_off(t + 1) - mv.D_off(t);
@@ -1947,7 +1960,7 @@ template <typename I, typename WT, int G, int NCH, bool FULL, bool PLAIN>
 int launch_bwd(const BwdArgs& a, SortWs& ws, uint32_t* chunk_start, int64_t N, hipStream_t s) {
   if (!ws.small) {
     if (int rc = prefix_scan_epi(
-            ChunkCount{a.cum}, N, reinterpret_cast<const int32_t*>(a.num_runs),
+            ChunkCount{a.cum, a.long_len}, N, reinterpret_cast<const int32_t*>(a.num_runs),
             ChunkEpi{a.cum, chunk_start, ws.chunk_mark, &ws.counters[1]}, scan_slot(ws, 1), s))
       return rc;
   }
@@ -2109,7 +2122,7 @@ int transpose_impl(const int64_t* hash_size_cumsum, int32_t T, int64_t B, const 
   if (workspace == nullptr || workspace_bytes < w.bytes)
     return set_error(MX_EWORKSPACE, "workspace of %zu bytes needed", w.bytes);
   TransposeOut o{linear_indices, sorted_linear_indices, infos_sorted, sorted_linear_indices_run,
-                 run_lengths, num_runs, cumulative_run_lengths, nullptr, nullptr};
+                 run_lengths, num_runs, cumulative_run_lengths, nullptr, nullptr, 0};
   w.small = small_batch(N, lay.nbags);
   return run_transpose(hash_size_cumsum, T, B, lay.nbags, lay.b_t_map, lay.B_offsets,
                        total_hash_size_bits,
@@ -2144,7 +2157,8 @@ int backward_impl(void* weights, int32_t weights_ty, const int64_t* weights_offs
     return set_error(MX_EWORKSPACE, "workspace of %zu bytes needed", w.bytes);
   auto* s = as_stream(stream);
   TransposeOut o{nullptr, w.sorted, w.infos, w.run, nullptr, nullptr, w.cum,
-                 indice_weights ? w.weights_sorted : nullptr, w.chunk_start};
+                 indice_weights ? w.weights_sorted : nullptr, w.chunk_start,
+                 long_run(T, max_D, total_D)};
   // A small batch uses no counters, so no region either.
   w.sort.small = small_batch(N, lay.nbags);
   ZeroedRegion* zr = w.sort.small ? nullptr : stream_region(s);
@@ -2184,6 +2198,7 @@ int backward_impl(void* weights, int32_t weights_ty, const int64_t* weights_offs
   a.nb = nb;
   a.pooling = pooling_mode;
   a.wd_mode = weight_decay_mode;
+  a.long_len = o.long_len;
   a.lr = learning_rate;
   a.eps = eps;
   a.wd = weight_decay;
