@@ -10,7 +10,7 @@ import torch
 import oracle as orc
 from mx_fbgemm import bench_inputs
 from adagrad_bounds import assert_eps_pin_close, assert_reordered_adagrad_close, eps_pin_case
-from tbe_helpers import random_tbe, weight_offsets
+from tbe_helpers import random_tbe, tbe_forward_gpu, weight_offsets
 
 pytestmark = pytest.mark.gpu
 
@@ -354,6 +354,46 @@ def test_grad_indice_weights(dev, pooling, dims):
             for t in np.flatnonzero(f == 0):
                 o = inp.offsets[t * inp.B], inp.offsets[(t + 1) * inp.B]
                 assert not got[o[0]:o[1]].any()
+
+
+@pytest.mark.parametrize("dims", [[68, 4, 256], [128, 36, 64], [260, 12, 512], [8, 516, 1024]])
+def test_mixed_width_weights(dev, dims):
+    """The mixed-width instances (by the widest table: up to 256, 512 and 1024
+    columns) of the weighted lookup and of its per-sample-weight gradient: a
+    narrow row's idle chunks take no part, so an infinite or NaN row shows in
+    its own positions alone."""
+    print(f"[case] mixed widths dims={dims}", flush=True)
+    T = len(dims)
+    rng = np.random.default_rng(sum(dims))
+    inp = random_tbe(rng, T, 45, dims, [60] * T, 20, empty_frac=0.1)
+    W = rng.uniform(-1, 1, size=sum(60 * D for D in dims)).astype(np.float32)
+    w_off = weight_offsets(inp)
+    for t, bad in enumerate((np.inf, np.nan, -np.inf)):  # row 1 + t of table t
+        W[w_off[t] + (1 + t) * dims[t]] = bad
+    table = np.repeat(np.arange(T), np.diff(inp.offsets[::inp.B]))
+    hit = inp.indices == 1 + table
+    assert hit.any() and not hit.all()
+    iw = rng.uniform(0.5, 2, size=inp.N).astype(np.float32)
+    grad = rng.normal(0, 1, size=(inp.B, inp.total_D)).astype(np.float32)
+    empty = torch.zeros(0, device=dev)
+    for wd in (W, W.astype(np.float16)):
+        got = tbe_forward_gpu(dev, torch.from_numpy(wd).to(dev), inp, 0,
+                              indice_weights=torch.from_numpy(iw)).cpu().numpy()
+        wf = wd.astype(np.float32)
+        exp = orc.tbe_forward_f32(wf, w_off, inp.D_offsets, inp.B, inp.indices, inp.offsets, 0, iw)
+        np.testing.assert_array_equal(got, exp)
+        g = torch.ops.fbgemm.split_embedding_codegen_grad_indice_weights_cuda(
+            torch.from_numpy(grad).to(dev), torch.from_numpy(wd).to(dev), empty, empty,
+            torch.zeros(T, dtype=torch.int32, device=dev), torch.from_numpy(w_off).to(dev),
+            torch.from_numpy(inp.D_offsets).to(dev), max(dims),
+            torch.from_numpy(inp.indices).to(dev), torch.from_numpy(inp.offsets).to(dev),
+            torch.zeros(0, dtype=torch.int32, device=dev), None, 0).cpu().numpy()
+        assert np.array_equal(np.isfinite(g), ~hit)
+        fin = np.where(np.isfinite(wf), wf, 0)
+        args = (w_off, inp.D_offsets, inp.B, inp.indices, inp.offsets, 0)
+        ref = orc.grad_indice_weights(grad, fin, *args)
+        mag = orc.grad_indice_weights(np.abs(grad), np.abs(fin), *args)
+        assert np.all(np.abs(g - ref)[~hit] <= 1e-5 * mag[~hit])
 
 
 @pytest.mark.parametrize("pooling", [0, 1])

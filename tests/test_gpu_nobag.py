@@ -235,11 +235,7 @@ def test_backward_nobag(dev, D, wd_mode, wd, dup):
     assert np.array_equal(Wg[untouched], W[untouched])
 
 
-@pytest.mark.parametrize("index_dtype", [torch.int64, torch.int32])
-def test_transpose_nobag(dev, index_dtype):
-    print(f"[case] nobag transpose idx={index_dtype}", flush=True)
-    rng = np.random.default_rng(17)
-    inp = random_tbe(rng, 4, 50, [8] * 4, [500, 30, 2000, 7], 25)
+def _check_transpose_nobag(dev, inp, index_dtype):
     out = torch.ops.fbgemm.transpose_embedding_input(
         torch.from_numpy(inp.hash_size_cumsum).to(dev), inp.total_hash_size_bits,
         torch.from_numpy(inp.indices).to(dev, index_dtype),
@@ -256,6 +252,41 @@ def test_transpose_nobag(dev, index_dtype):
     np.testing.assert_array_equal(lengths[:r], exp["run_lengths"])
     np.testing.assert_array_equal(cum[:r + 1], exp["cumulative_run_lengths"])
     assert np.all(lengths[r:] == 0) and np.all(cum[r + 1:] == inp.N)
+
+
+@pytest.mark.parametrize("index_dtype", [torch.int64, torch.int32])
+def test_transpose_nobag(dev, index_dtype):
+    print(f"[case] nobag transpose idx={index_dtype}", flush=True)
+    rng = np.random.default_rng(17)
+    inp = random_tbe(rng, 4, 50, [8] * 4, [500, 30, 2000, 7], 25)
+    _check_transpose_nobag(dev, inp, index_dtype)
+
+
+@pytest.mark.parametrize("T,B,D", [(1, 700, 12), (1, 1100, 12), (63, 20, 96), (63, 60, 96),
+                                   (64, 20, 36), (64, 60, 36), (1025, 2, 4), (1025, 6, 4)])
+def test_sequence_batch_sizes(dev, T, B, D):
+    """The transpose (bit-exact) and the update of sequence batches either side
+    of 8192 positions (one block or the chain), with tables either side of the
+    63 that may sort as segments and of the 1024 whose first positions are
+    staged, empty tables included, at widths that leave lanes idle."""
+    print(f"[case] sequence batch T={T} B={B} D={D}", flush=True)
+    rng = np.random.default_rng(T + B)
+    rows = [int(r) for r in rng.integers(1, 9 if T > 1 else 4000, T)]
+    inp = random_tbe(rng, T, B, [D] * T, rows, 8 if T > 1 else 25, empty_frac=0.3)
+    assert (inp.N > 8192) == (B in (1100, 60, 6)), inp.N
+    _check_transpose_nobag(dev, inp, torch.int64)
+    W = rng.uniform(-0.5, 0.5, size=sum(E * D for E in rows)).astype(np.float32)
+    m1 = rng.uniform(0, 0.01, size=sum(rows)).astype(np.float32)
+    m1_off = np.concatenate([[0], np.cumsum(rows)[:-1]]).astype(np.int64)
+    grad = rng.normal(0, 0.01, size=(inp.N, D)).astype(np.float32)
+    Wd, m1d = torch.from_numpy(W).to(dev), torch.from_numpy(m1).to(dev)
+    _backward_nobag(dev, Wd, m1d, m1_off, inp, D, grad, 0.05, 1e-8, 0.02, 1, torch.int64)
+    W_exp, m_exp = orc.backward_rowwise_adagrad_nobag(
+        W, weight_offsets(inp), D, B, inp.hash_size_cumsum, inp.total_hash_size_bits,
+        inp.indices, inp.offsets, grad, m1, m1_off, 0.05, 1e-8, 0.02, 1)
+    # Long runs sum their rows in chunks: the bounds of the duplicate-heavy case above.
+    np.testing.assert_allclose(m1d.cpu().numpy(), m_exp, rtol=1e-4, atol=0)
+    np.testing.assert_allclose(Wd.cpu().numpy(), W_exp, rtol=RTOL, atol=1e-6)
 
 
 def test_training_module_nobag_step(dev):
@@ -358,7 +389,7 @@ def test_nobag_sort_segments(dev, layout):
     W_exp, m_exp = orc.backward_rowwise_adagrad_nobag(
         W, w_off, D, B, hsc, bits, indices, offsets, grad, m1, m1_off, lr, eps)
     Wg, mg = Wd.cpu().numpy(), m1d.cpu().numpy()
-    # Runs past 24 occurrences sum in 32-row chunks: another association of the terms.
+    # Long runs sum in 32-row chunks: another association of the terms.
     np.testing.assert_allclose(mg, m_exp, rtol=1e-4, atol=0)
     np.testing.assert_allclose(Wg, W_exp, rtol=RTOL, atol=1e-6)
     untouched = W_exp == W

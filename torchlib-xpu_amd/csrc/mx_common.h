@@ -101,6 +101,9 @@ __device__ __forceinline__ float fp32_value(float v) {
   return v;
 }
 
+// Waits for every vector load of the wave (vmcnt 0, the other counts free).
+__device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0f70); }
+
 // Sum over all 64 lanes (tree order fixed: deterministic).
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll

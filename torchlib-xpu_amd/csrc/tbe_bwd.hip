@@ -141,7 +141,27 @@ struct SegSort {
 // [w * kLinTile / 4, (w + 1) * kLinTile / 4), 64 consecutive ones per item.
 constexpr int kLinWavePos = kLinTile / 4;
 
-template <typename I>
+// Sequence batches (PoolingMode NONE): tables whose first positions fit LDS.
+constexpr int kNobagMaxT = 1024;
+
+// The table of position l: the last t with first(t) <= l.
+template <class First>
+__device__ __forceinline__ int32_t seq_table(int64_t l, int32_t T, First first) {
+  int32_t lo = 0, hi = T;
+  while (hi - lo > 1) {
+    const int32_t mid = lo + ((hi - lo) >> 1);
+    if (first(mid) <= l)
+      lo = mid;
+    else
+      hi = mid;
+  }
+  return lo;
+}
+
+// SEQ: a sequence batch, in which every position is a bag of its own: table t's
+// positions start at offsets[t * seq_B], a position's info word holds t and its
+// place among them, and no bag is searched.
+template <typename I, bool SEQ>
 __global__ void __launch_bounds__(256)
     linearize_kernel(const int64_t* __restrict__ hsc, const I* __restrict__ indices,
                      const I* __restrict__ offsets, int64_t nbags, int64_t B, int32_t nb,
@@ -150,7 +170,7 @@ __global__ void __launch_bounds__(256)
                      uint32_t* __restrict__ keys, uint32_t* __restrict__ vals,
                      const float* __restrict__ iw, uint32_t* __restrict__ vals2,
                      uint32_t* __restrict__ ghist, unsigned long long* __restrict__ zero,
-                     int64_t zero_words, SegSort seg) {
+                     int64_t zero_words, SegSort seg, int32_t T, int64_t seq_B) {
   __shared__ uint32_t s_mark[kLinTile];  // bag (relative to blo) starting at each position
   __shared__ uint32_t hf[2][kMaxPasses][kRadix];  // digit counts of the block's first two features
   __shared__ int s_bad;
@@ -165,6 +185,11 @@ __global__ void __launch_bounds__(256)
   __shared__ uint32_t s_cnt[2][2];       // [half][wave of the half]
   __shared__ uint32_t s_wmax[4];
   __shared__ uint32_t h[kMaxPasses][kRadix];
+  __shared__ int64_t s_first[SEQ ? kNobagMaxT + 1 : 1];  // first position of each table
+  const bool first_lds = T <= kNobagMaxT;
+  auto first = [&](int64_t t) -> int64_t {
+    return SEQ && first_lds ? s_first[t] : static_cast<int64_t>(offsets[t * seq_B]);
+  };
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int64_t l0 = static_cast<int64_t>(blockIdx.x) * kLinTile;
   const int64_t lend = l0 + kLinTile < N ? l0 + kLinTile : N;
@@ -183,12 +208,18 @@ __global__ void __launch_bounds__(256)
   // after the searches, when it has arrived.
   const int64_t lane_hsc = seg.T > 0 && w == 0 && lane <= seg.T ? hsc[lane] : 0;
   const int32_t lane_boff = seg.B_off && w == 0 && lane <= seg.T ? seg.B_off[lane] : 0;
+  if constexpr (SEQ) {
+    if (first_lds)
+      for (int t = threadIdx.x; t <= T; t += 256) s_first[t] = static_cast<int64_t>(offsets[t * seq_B]);
+    if (threadIdx.x < 2) s_range[threadIdx.x][0] = 0;
+    __syncthreads();
+  }
   // Last bag with offsets[bag] <= target (0 when none), for the block's first
   // (half 0) and last (half 1) position: 128-ary searches, one probe per
   // thread and round, so ceil(log128(nbags)) dependent loads instead of
   // log2(nbags).  Invariant: offsets[lo] <= target < offsets[hi] (hi = nbags:
   // past the end).
-  {
+  if constexpr (!SEQ) {
     const int half = threadIdx.x >> 7, q = threadIdx.x & 127;
     const int64_t target = half == 0 ? l0 : lend - 1;
     if (q == 0) {
@@ -260,7 +291,9 @@ __global__ void __launch_bounds__(256)
   // The block's first feature: its first bag's (checked below for a variable
   // batch, whose bags need not match a feature's B_off range).
   int64_t t_lo = 0;
-  if (seg.T > 0) {
+  if constexpr (SEQ) {
+    t_lo = seq_table(l0, T, first);
+  } else if (seg.T > 0) {
     t_lo = seg.B_off ? (nb >= 32 ? 0 : static_cast<int64_t>(static_cast<uint32_t>(b_t_map[blo]) >> nb))
                      : blo / B;
     if (t_lo >= seg.T) t_lo = seg.T - 1;
@@ -271,8 +304,15 @@ __global__ void __launch_bounds__(256)
   // largest mark at or before l (an inclusive max-scan; bag ids grow with
   // position, and position l0 belongs to bag blo, mark 0).
   const bool marked = bhi - blo < 4 * kLinTile;  // block-uniform
-  uint32_t rel[kLinItems];
-  if (marked) {
+  uint32_t rel[kLinItems];  // SEQ: the position's table
+  if constexpr (SEQ) {
+#pragma unroll
+    for (int it = 0; it < kLinItems; ++it) {
+      const int64_t l = pbase + it * 64;
+      rel[it] = l < lend ? static_cast<uint32_t>(seq_table(l, T, first)) : 0u;
+    }
+    __syncthreads();  // count arrays cleared
+  } else if (marked) {
     for (int i = threadIdx.x; i < kLinTile; i += 256) s_mark[i] = 0u;
     __syncthreads();
     for (int64_t b = blo + threadIdx.x; b <= bhi; b += 256) {
@@ -333,7 +373,11 @@ __global__ void __launch_bounds__(256)
       // Info word (t << nb) | b: computed for a fixed batch, given per bag (VBE).
       uint32_t info;
       int64_t t;
-      if (b_t_map) {
+      if constexpr (SEQ) {
+        t = rel[it];
+        const int64_t b = l - first(t) > 0 ? l - first(t) : 0;
+        info = (nb >= 32 ? 0u : (rel[it] << nb)) | static_cast<uint32_t>(b);
+      } else if (b_t_map) {
         info = static_cast<uint32_t>(b_t_map[bag]);
         t = nb >= 32 ? 0 : static_cast<int64_t>(info >> nb);
       } else {
@@ -343,7 +387,7 @@ __global__ void __launch_bounds__(256)
       }
       // A variable batch's segments take their positions from B_off, so each
       // bag must lie in its own feature's range of bags; else the sort is global.
-      if (seg.B_off && (t >= seg.T || bag < s_boff[t] || bag >= s_boff[t + 1])) {
+      if (!SEQ && seg.B_off && (t >= seg.T || bag < s_boff[t] || bag >= s_boff[t + 1])) {
         s_bad = 1;
         if (t >= seg.T) t = seg.T - 1;  // in-bounds LDS reads
       }
@@ -395,7 +439,9 @@ __global__ void __launch_bounds__(256)
         int64_t fbag = seg.B_off ? static_cast<int64_t>(s_boff[s_gfirst[lane < S ? lane : S]])
                                  : static_cast<int64_t>(s_gfirst[lane < S ? lane : S]) * B;
         fbag = fbag < 0 ? 0 : (fbag > nbags ? nbags : fbag);  // a bad B_off fails the checks below
-        const int64_t fp = lane <= S ? static_cast<int64_t>(offsets[fbag]) : N;
+        const int64_t fp = lane > S ? N
+                           : SEQ    ? first(s_gfirst[lane])
+                                    : static_cast<int64_t>(offsets[fbag]);
         const int64_t fnext = __shfl(fp, lane + 1 < 64 ? lane + 1 : 63, 64);
         const uint32_t nt = lane < S ? static_cast<uint32_t>(ceil_div(fnext - fp, kSweepTile)) : 0u;
         const uint32_t incl = wave_incl_scan<SumOp>(nt);
@@ -885,6 +931,8 @@ struct SmallSort {
   uint32_t* total_chunks;
   int32_t max_chunks;     // entries of chunk_mark
   uint32_t long_len;      // runs longer than this are chunked
+  int32_t T;              // with seq_B: a sequence batch, as in linearize; 0: bags
+  int64_t seq_B;
 };
 
 // Sum over the block's waves before this one, and over all; a barrier on entry
@@ -928,8 +976,9 @@ __global__ void __launch_bounds__(kSweepThreads) small_transpose_kernel(SmallSor
   if (threadIdx.x == 0 && a.fail) *a.fail = 0u;
   __syncthreads();
   // Each non-empty bag marks its first position (0: bag 0, as before any bag).
+  const int64_t marking = a.seq_B ? 0 : a.nbags;
 #pragma unroll 4
-  for (int64_t b = threadIdx.x; b < a.nbags; b += kSweepThreads) {
+  for (int64_t b = threadIdx.x; b < marking; b += kSweepThreads) {
     const int64_t o0 = static_cast<int64_t>(offsets[b]);
     const int64_t o1 = static_cast<int64_t>(offsets[b + 1]);
     if (o1 > o0 && o0 >= 0 && o0 < N) s_key[o0] = static_cast<uint32_t>(b);
@@ -963,7 +1012,13 @@ __global__ void __launch_bounds__(kSweepThreads) small_transpose_kernel(SmallSor
       if (i >= N) continue;
       uint32_t info;
       int64_t t;
-      if (a.b_t_map) {
+      if (a.seq_B) {
+        auto first = [&](int64_t x) { return static_cast<int64_t>(offsets[x * a.seq_B]); };
+        const int32_t ts = seq_table(i, a.T, first);
+        const int64_t b = i - first(ts) > 0 ? i - first(ts) : 0;
+        t = ts;
+        info = (a.nb >= 32 ? 0u : (static_cast<uint32_t>(ts) << a.nb)) | static_cast<uint32_t>(b);
+      } else if (a.b_t_map) {
         info = static_cast<uint32_t>(a.b_t_map[bag]);
         t = a.nb >= 32 ? 0 : static_cast<int64_t>(info >> a.nb);
       } else {
@@ -1319,11 +1374,13 @@ ZeroedRegion* stream_region(hipStream_t s) {
 }
 
 // nbags = T * B bags of a fixed batch B, or (b_t_map non-null, VBE) the
-// total bag count with each bag's info word given.  zr: the stream's zeroed
+// total bag count with each bag's info word given, or (seq_B > 0) a sequence
+// batch of N positions in bags of batch seq_B.  zr: the stream's zeroed
 // region for the early words (held locked by the caller, whose last kernel
 // clears w.early_words of it), or null: the workspace's, cleared here.
 int run_transpose(const int64_t* hsc, int32_t T, int64_t B, int64_t nbags,
-                  const int32_t* b_t_map, const int32_t* B_off, int32_t bits, int32_t nb, const void* indices,
+                  const int32_t* b_t_map, const int32_t* B_off, int64_t seq_B, int32_t bits,
+                  int32_t nb, const void* indices,
                   const void* offsets, int32_t index_bytes, int64_t N, const float* iw,
                   const TransposeOut& o, SortWs& w, hipStream_t s, ZeroedRegion* zr) {
   // With per-sample weights the weights travel with the keys as a second payload.
@@ -1337,7 +1394,8 @@ int run_transpose(const int64_t* hsc, int32_t T, int64_t B, int64_t nbags,
                       o.linear, iw, w.vals[0], o.sorted, reinterpret_cast<uint32_t*>(o.infos),
                       o.weights_sorted, o.run, o.cum, o.run_lengths, o.num_runs, &w.counters[0],
                       w.fail, o.chunk_start, chunks ? w.chunk_mark : nullptr, &w.counters[1],
-                      static_cast<int32_t>(max_chunks(N)), static_cast<uint32_t>(o.long_len)};
+                      static_cast<int32_t>(max_chunks(N)), static_cast<uint32_t>(o.long_len), T,
+                      seq_B};
     return index_bytes == 8 ? launch_small_transpose<int64_t>(a, s)
                             : launch_small_transpose<int32_t>(a, s);
   }
@@ -1370,16 +1428,17 @@ int run_transpose(const int64_t* hsc, int32_t T, int64_t B, int64_t nbags,
   // Linearize also clears the look-back state of the later kernels.
   const int64_t late_words = late_zeroed_words(w, passes, pass_words);
   const dim3 glin(static_cast<uint32_t>(ceil_div(N, kLinTile)));
+  auto linearize = [&](auto i0, auto seq) {
+    using I = decltype(i0);
+    linearize_kernel<I, decltype(seq)::value><<<glin, 256, 0, s>>>(
+        hsc, static_cast<const I*>(indices), static_cast<const I*>(offsets), nbags, B, nb, b_t_map,
+        N, bits, passes, o.linear, w.keys[0], w.vals[0], iw, v2[0], w.ghist, w.late, late_words,
+        seg, T, seq_B);
+  };
   if (index_bytes == 8)
-    linearize_kernel<int64_t><<<glin, 256, 0, s>>>(
-        hsc, static_cast<const int64_t*>(indices), static_cast<const int64_t*>(offsets), nbags, B,
-        nb, b_t_map, N, bits, passes, o.linear, w.keys[0], w.vals[0], iw, v2[0], w.ghist,
-        w.late, late_words, seg);
+    seq_B > 0 ? linearize(int64_t{}, std::true_type{}) : linearize(int64_t{}, std::false_type{});
   else
-    linearize_kernel<int32_t><<<glin, 256, 0, s>>>(
-        hsc, static_cast<const int32_t*>(indices), static_cast<const int32_t*>(offsets), nbags, B,
-        nb, b_t_map, N, bits, passes, o.linear, w.keys[0], w.vals[0], iw, v2[0], w.ghist,
-        w.late, late_words, seg);
+    seq_B > 0 ? linearize(int32_t{}, std::true_type{}) : linearize(int32_t{}, std::false_type{});
   MX_LAUNCH_CHECK();
 
   const dim3 gsweep(static_cast<uint32_t>(ntiles));
@@ -1441,6 +1500,7 @@ struct BwdArgs {
   const float* iw_sorted;  // per-sample weights in sorted order, or null
   const int32_t* B_off;    // VBE: first bag of each table [T+1], or null (fixed batch)
   const int64_t* row_out;  // VBE: gradient row offset of each bag, or null
+  int64_t seq_B;           // sequence batch: position offsets[t * seq_B] + b has row * max_D; else 0
   const uint32_t* num_runs;
   const uint32_t* chunk_start;
   const uint32_t* chunk_mark;  // chunk marks (kMarkEvery), from the chunk-count scan
@@ -1490,7 +1550,7 @@ struct TableMeta {
 __device__ __forceinline__ void stage_meta(const BwdArgs& a, TableMeta& m) {
   if (a.T <= kMaxCachedTables) {
     for (int i = threadIdx.x; i <= a.T; i += blockDim.x) {
-      m.D_off[i] = a.D_off[i];
+      m.D_off[i] = a.D_off ? a.D_off[i] : i * a.max_D;  // null: every table max_D wide
       if (i < a.T) {
         m.hsc[i] = a.hsc[i];
         m.w_off[i] = a.w_off[i];
@@ -1508,7 +1568,9 @@ struct MetaView {
   __device__ int64_t hsc(int64_t t) const { return cached ? m.hsc[t] : a.hsc[t]; }
   __device__ int64_t w_off(int64_t t) const { return cached ? m.w_off[t] : a.w_off[t]; }
   __device__ int64_t m1_off(int64_t t) const { return cached ? m.m1_off[t] : a.m1_off[t]; }
-  __device__ int32_t D_off(int64_t t) const { return cached ? m.D_off[t] : a.D_off[t]; }
+  __device__ int32_t D_off(int64_t t) const {
+    return cached ? m.D_off[t] : (a.D_off ? a.D_off[t] : static_cast<int32_t>(t) * a.max_D);
+  }
 };
 
 __device__ __forceinline__ void ld4(const float* p, float (&v)[4]) {
@@ -1555,19 +1617,30 @@ __device__ __forceinline__ bool col_in(int c, int k, int32_t D) {
   return FULL || (c * G + k) * 4 < D;
 }
 
+// The column that lane k loads for chunk c: its own, or the row's first ones where
+// the chunk lies past the row (unused there: not summed into h, not stored), so
+// that no load sits behind a branch, where an fp16 row waited for each chunk.
+template <bool FULL, int G>
+__device__ __forceinline__ int load_col(int c, int k, int32_t D) {
+  return col_in<FULL, G>(c, k, D) ? (c * G + k) * 4 : 0;
+}
+
 // A plain instance serves the common call -- SUM pooling, no per-sample
 // weights, a fixed batch, no weight decay -- with those options as
 // constants, so every per-element test on them folds away (config 3: update
-// launch 66.7 -> 62.6 us, chunk sums 16.0 -> 14.5 us).
-template <bool PLAIN>
+// launch 66.7 -> 62.6 us, chunk sums 16.0 -> 14.5 us).  A sequence instance
+// does the same for PoolingMode NONE (weight decay at run time).
+constexpr int kGeneral = 0, kPlain = 1, kSeq = 2;
+template <int MODE>
 __device__ __forceinline__ void pin_options(BwdArgs& a) {
-  if constexpr (PLAIN) {
+  if constexpr (MODE != kGeneral) {
     a.pooling = MX_POOL_SUM;
     a.iw_sorted = nullptr;
     a.B_off = nullptr;
     a.row_out = nullptr;
-    a.wd_mode = 0;
   }
+  if constexpr (MODE == kPlain) a.wd_mode = 0;
+  if constexpr (MODE != kSeq) a.seq_B = 0;
 }
 
 // Group-level (G lanes, lane k) sum of the (MEAN-scaled) gradient rows of
@@ -1597,7 +1670,11 @@ __device__ void group_sum_occurrences(const BwdArgs& a, const MetaView& mv, int3
       const int64_t bag = a.B_off ? a.B_off[tj] + b : tj * a.B + b;
       // Full width: every feature's columns start at tj * G*NCH*4 (config 3:
       // chunk sums 14.5 -> 12.8 us against the table lookup).
-      my_row = a.row_out ? a.row_out[bag] : b * a.total_D + (FULL ? tj * (G * NCH * 4) : mv.D_off(tj));
+      if (a.seq_B)
+        my_row = (static_cast<int64_t>(static_cast<const I*>(a.offsets)[tj * a.seq_B]) + b) * a.max_D;
+      else
+        my_row = a.row_out ? a.row_out[bag]
+                           : b * a.total_D + (FULL ? tj * (G * NCH * 4) : mv.D_off(tj));
       if (a.pooling == MX_POOL_MEAN) {
         const I* off = static_cast<const I*>(a.offsets);
         const int64_t L = static_cast<int64_t>(off[bag + 1]) - static_cast<int64_t>(off[bag]);
@@ -1613,10 +1690,15 @@ __device__ void group_sum_occurrences(const BwdArgs& a, const MetaView& mv, int3
         if (j + u < n) {
           const float* row = a.grad + __shfl(my_row, g * G + j + u, 64);
 #pragma unroll
-          for (int c = 0; c < NCH; ++c)
-            if (col_in<FULL, G>(c, k, D)) ld4(row + (c * G + k) * 4, v[u][c]);
+          for (int c = 0; c < NCH; ++c) ld4(row + load_col<FULL, G>(c, k, D), v[u][c]);
         }
       }
+      // All U rows have arrived from here on.  The sums wait for them anyway; said
+      // outright, no load is pending at the loop's end on any path, where the
+      // compiler otherwise waits before every load of the next round, in case an
+      // earlier one into its registers is still in flight (96-column sequences:
+      // chunk sums 41 us, 20).
+      wait_loads();
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         if (j + u < n) {
@@ -1624,14 +1706,12 @@ __device__ void group_sum_occurrences(const BwdArgs& a, const MetaView& mv, int3
           const float wt = __shfl(my_w, g * G + j + u, 64);
 #pragma unroll
           for (int c = 0; c < NCH; ++c)
-            if (col_in<FULL, G>(c, k, D)) {
 #pragma unroll
-              for (int e = 0; e < 4; ++e) {
-                float x = v[u][c][e];
-                if (mean) x = __fmul_rn(x, sc);
-                if (weighted) x = __fmul_rn(x, wt);
-                acc[c][e] += x;
-              }
+            for (int e = 0; e < 4; ++e) {
+              float x = v[u][c][e];
+              if (mean) x = __fmul_rn(x, sc);
+              if (weighted) x = __fmul_rn(x, wt);
+              acc[c][e] += x;
             }
         }
       }
@@ -1782,8 +1862,7 @@ __device__ __forceinline__ void long_run_body(const BwdArgs& a, const MetaView& 
       float h0 = 0.0f;
       if (grp == 0) {  // the row and its momentum load while the partials are summed
 #pragma unroll
-        for (int c = 0; c < NCH; ++c)
-          if (col_in<FULL, G>(c, k, D)) ld_row4(wrow + (c * G + k) * 4, w[c]);
+        for (int c = 0; c < NCH; ++c) ld_row4(wrow + load_col<FULL, G>(c, k, D), w[c]);
         h0 = *hp;
       }
       float gs[NCH][4];
@@ -1798,15 +1877,14 @@ __device__ __forceinline__ void long_run_body(const BwdArgs& a, const MetaView& 
           if (qq + u * NG < q1)
 #pragma unroll
             for (int c = 0; c < NCH; ++c)
-              if (col_in<FULL, G>(c, k, D)) ld4(a.partial + (qq + u * NG) * a.max_D + (c * G + k) * 4, v[u][c]);
+              ld4(a.partial + (qq + u * NG) * a.max_D + load_col<FULL, G>(c, k, D), v[u][c]);
 #pragma unroll
         for (int u = 0; u < U; ++u)
           if (qq + u * NG < q1)
 #pragma unroll
             for (int c = 0; c < NCH; ++c)
-              if (col_in<FULL, G>(c, k, D))
 #pragma unroll
-                for (int e = 0; e < 4; ++e) gs[c][e] += v[u][c][e];
+              for (int e = 0; e < 4; ++e) gs[c][e] += v[u][c][e];
       }
 #pragma unroll
       for (int c = 0; c < NCH; ++c)
@@ -1840,9 +1918,9 @@ __device__ __forceinline__ void long_run_body(const BwdArgs& a, const MetaView& 
 }
 
 // Pass A: one group per chunk of a long run -> partial sum in the workspace.
-template <typename I, int G, int NCH, int U, bool FULL, bool PLAIN>
+template <typename I, int G, int NCH, int U, bool FULL, int MODE>
 __global__ void __launch_bounds__(256) bwd_chunk_kernel(BwdArgs a) {
-  pin_options<PLAIN>(a);
+  pin_options<MODE>(a);
   if (call_failed(a.fail)) return;  // the run layout is not valid
   __shared__ TableMeta meta;
   stage_meta(a, meta);
@@ -1906,8 +1984,7 @@ __device__ __forceinline__ void short_run_body(const BwdArgs& a, const MetaView&
     float* hp = a.m1 + mv.m1_off(t) + idx;
     float w[NCH][4];
 #pragma unroll
-    for (int c = 0; c < NCH; ++c)
-      if (col_in<FULL, G>(c, k, D)) ld_row4(wrow + (c * G + k) * 4, w[c]);
+    for (int c = 0; c < NCH; ++c) ld_row4(wrow + load_col<FULL, G>(c, k, D), w[c]);
     const float h0 = *hp;
     float gs[NCH][4];
 #pragma unroll
@@ -1935,7 +2012,7 @@ constexpr int runs_waves() {
 }
 
 template <typename I, typename WT, int G, int NCH, int U, int GL, int NCHL, int UL, bool FULL,
-          bool PLAIN>
+          int MODE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(runs_waves<NCH>())))
     bwd_runs_kernel(BwdArgs a, int64_t nlong) {
   // The early words go back to zero for the stream's next call, also when
@@ -1943,7 +2020,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(runs_w
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < a.rezero_words;
        i += static_cast<int64_t>(gridDim.x) * 256)
     a.rezero[i] = 0ull;
-  pin_options<PLAIN>(a);
+  pin_options<MODE>(a);
   if (call_failed(a.fail)) return;  // the run layout is not valid
   __shared__ TableMeta meta;
   stage_meta(a, meta);
@@ -1956,7 +2033,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(runs_w
 
 // After the run encoding: the chunk layout of the long runs (chunk-count
 // scan), their chunk partial sums, then both run classes in one launch.
-template <typename I, typename WT, int G, int NCH, bool FULL, bool PLAIN>
+template <typename I, typename WT, int G, int NCH, bool FULL, int MODE>
 int launch_bwd(const BwdArgs& a, SortWs& ws, uint32_t* chunk_start, int64_t N, hipStream_t s) {
   if (!ws.small) {
     if (int rc = prefix_scan_epi(
@@ -1970,7 +2047,7 @@ int launch_bwd(const BwdArgs& a, SortWs& ws, uint32_t* chunk_start, int64_t N, h
   const int64_t nblk = want < 1 ? 1 : (want > cus * 16 ? cus * 16 : want);
   const int64_t ngrid = ceil_div(nblk, 8) * 8;  // whole rounds over the XCDs
   constexpr int UC = NCH <= 1 ? 8 : (NCH <= 2 ? 8 : 4);  // chunks are full: more in flight
-  bwd_chunk_kernel<I, G, NCH, UC, FULL, PLAIN><<<dim3(static_cast<uint32_t>(ngrid)), 256, 0, s>>>(a);
+  bwd_chunk_kernel<I, G, NCH, UC, FULL, MODE><<<dim3(static_cast<uint32_t>(ngrid)), 256, 0, s>>>(a);
   MX_LAUNCH_CHECK();
   // Long runs: twice the lanes per row where the row allows (more groups
   // summing partials per block; measured 15.1 -> 12.4 us on config 3).
@@ -1981,7 +2058,7 @@ int launch_bwd(const BwdArgs& a, SortWs& ws, uint32_t* chunk_start, int64_t N, h
   const int64_t long_cap = cus * kLongBlocksPerCu;
   const int64_t nlong = ceil_div(long_want < long_cap ? long_want : long_cap, 8) * 8;
   constexpr int UL = NCHL <= 1 ? 4 : (NCHL <= 2 ? 2 : 1);  // 64 bytes per lane in flight
-  bwd_runs_kernel<I, WT, G, NCH, U, GL, NCHL, UL, FULL, PLAIN>
+  bwd_runs_kernel<I, WT, G, NCH, U, GL, NCHL, UL, FULL, MODE>
       <<<dim3(static_cast<uint32_t>(nlong + ngrid)), 256, 0, s>>>(a, nlong);
   MX_LAUNCH_CHECK();
   return MX_OK;
@@ -1998,11 +2075,16 @@ int launch_width(const BwdArgs& a, SortWs& ws, uint32_t* chunk_start, int64_t N,
   const bool full = a.max_D == kWidth && a.total_D == static_cast<int64_t>(a.T) * kWidth;
   const bool plain = a.pooling == MX_POOL_SUM && a.iw_sorted == nullptr && a.B_off == nullptr &&
                      a.wd_mode == 0;
-  if (full)
-    return plain ? launch_bwd<I, WT, G, NCH, true, true>(a, ws, chunk_start, N, s)
-                 : launch_bwd<I, WT, G, NCH, true, false>(a, ws, chunk_start, N, s);
-  return plain ? launch_bwd<I, WT, G, NCH, false, true>(a, ws, chunk_start, N, s)
-               : launch_bwd<I, WT, G, NCH, false, false>(a, ws, chunk_start, N, s);
+  auto go = [&](auto full_c, auto mode) {
+    return launch_bwd<I, WT, G, NCH, decltype(full_c)::value, decltype(mode)::value>(
+        a, ws, chunk_start, N, s);
+  };
+  auto by_mode = [&](auto full_c) {
+    if (a.seq_B) return go(full_c, std::integral_constant<int, kSeq>{});
+    return plain ? go(full_c, std::integral_constant<int, kPlain>{})
+                 : go(full_c, std::integral_constant<int, kGeneral>{});
+  };
+  return full ? by_mode(std::true_type{}) : by_mode(std::false_type{});
 }
 
 // Lanes per run (G) and float4 chunks per lane (NCH) from the widest table.
@@ -2083,6 +2165,7 @@ struct Layout {
   const int32_t* B_offsets;
   const int64_t* row_out;
   const int32_t* b_t_map;
+  int64_t seq_B;  // sequence batch: its batch size; else 0
 };
 
 int check_common(int32_t T, int64_t B, const Layout& lay, int32_t bits, int32_t nb,
@@ -2124,7 +2207,7 @@ int transpose_impl(const int64_t* hash_size_cumsum, int32_t T, int64_t B, const 
   TransposeOut o{linear_indices, sorted_linear_indices, infos_sorted, sorted_linear_indices_run,
                  run_lengths, num_runs, cumulative_run_lengths, nullptr, nullptr, 0};
   w.small = small_batch(N, lay.nbags);
-  return run_transpose(hash_size_cumsum, T, B, lay.nbags, lay.b_t_map, lay.B_offsets,
+  return run_transpose(hash_size_cumsum, T, B, lay.nbags, lay.b_t_map, lay.B_offsets, lay.seq_B,
                        total_hash_size_bits,
                        info_B_num_bits, indices, offsets, index_bytes, N, nullptr, o, w, s,
                        nullptr);
@@ -2149,7 +2232,7 @@ int backward_impl(void* weights, int32_t weights_ty, const int64_t* weights_offs
   MX_REQUIRE(weights_ty == MX_SPARSE_FP32 || weights_ty == MX_SPARSE_FP16,
              "weights type %d not supported (FP32=0, FP16=1)", weights_ty);
   if (N == 0) return MX_OK;
-  MX_REQUIRE(weights && weights_offsets && D_offsets && hash_size_cumsum && indices && offsets &&
+  MX_REQUIRE(weights && weights_offsets && (D_offsets || lay.seq_B) && hash_size_cumsum && indices && offsets &&
                  grad_output && momentum1 && momentum1_offsets,
              "null pointer argument");
   BwdWs w = carve_bwd(static_cast<uint8_t*>(workspace), N, max_D);
@@ -2164,7 +2247,7 @@ int backward_impl(void* weights, int32_t weights_ty, const int64_t* weights_offs
   ZeroedRegion* zr = w.sort.small ? nullptr : stream_region(s);
   std::unique_lock<std::mutex> zr_lock;
   if (zr) zr_lock = std::unique_lock<std::mutex>(zr->mu);
-  if (int rc = run_transpose(hash_size_cumsum, T, B, lay.nbags, lay.b_t_map, lay.B_offsets,
+  if (int rc = run_transpose(hash_size_cumsum, T, B, lay.nbags, lay.b_t_map, lay.B_offsets, lay.seq_B,
                              total_hash_size_bits, nb, indices, offsets, index_bytes, N,
                              indice_weights, o, w.sort, s, zr))
     return rc;
@@ -2185,6 +2268,7 @@ int backward_impl(void* weights, int32_t weights_ty, const int64_t* weights_offs
   a.iw_sorted = indice_weights ? w.weights_sorted : nullptr;
   a.B_off = lay.b_t_map ? lay.B_offsets : nullptr;
   a.row_out = lay.b_t_map ? lay.row_out : nullptr;
+  a.seq_B = lay.seq_B;
   a.num_runs = &w.sort.counters[0];
   a.chunk_start = w.chunk_start;
   a.chunk_mark = w.sort.chunk_mark;
@@ -2228,7 +2312,7 @@ extern "C" int mx_tbe_transpose_embedding_input(
     int64_t* sorted_linear_indices_run, int32_t* run_lengths, int32_t* num_runs,
     int32_t* cumulative_run_lengths, void* workspace, size_t workspace_bytes, void* stream) {
   clear_error();
-  const Layout lay{static_cast<int64_t>(T) * B, nullptr, nullptr, nullptr};
+  const Layout lay{static_cast<int64_t>(T) * B, nullptr, nullptr, nullptr, 0};
   return transpose_impl(hash_size_cumsum, T, B, lay, total_hash_size_bits, info_B_num_bits,
                         indices, offsets, index_bytes, N, linear_indices, sorted_linear_indices,
                         infos_sorted, sorted_linear_indices_run, run_lengths, num_runs,
@@ -2245,7 +2329,7 @@ extern "C" int mx_tbe_transpose_embedding_input_vbe(
   clear_error();
   MX_REQUIRE(total_B == 0 || vbe_b_t_map, "VBE needs the b_t map");
   // Sorting needs only each bag's info word.
-  const Layout lay{total_B, nullptr, nullptr, vbe_b_t_map};
+  const Layout lay{total_B, nullptr, nullptr, vbe_b_t_map, 0};
   return transpose_impl(hash_size_cumsum, T, 0, lay, total_hash_size_bits, info_B_num_bits,
                         indices, offsets, index_bytes, N, linear_indices, sorted_linear_indices,
                         infos_sorted, sorted_linear_indices_run, run_lengths, num_runs,
@@ -2269,7 +2353,7 @@ extern "C" int mx_tbe_backward_rowwise_adagrad(
   clear_error();
   const int32_t nb = mx_tbe_info_B_num_bits(T, B);
   MX_REQUIRE(nb > 0, "T=%d, B=%lld do not fit a 32-bit info word", T, (long long)B);
-  const Layout lay{static_cast<int64_t>(T) * B, nullptr, nullptr, nullptr};
+  const Layout lay{static_cast<int64_t>(T) * B, nullptr, nullptr, nullptr, 0};
   return backward_impl(weights, weights_ty, weights_offsets, D_offsets, T, B, nb, lay, max_D,
                        hash_size_cumsum, total_hash_size_bits, indices, offsets, index_bytes, N,
                        pooling_mode, indice_weights, grad_output, total_D, momentum1,
@@ -2290,7 +2374,7 @@ extern "C" int mx_tbe_backward_rowwise_adagrad_vbe(
   clear_error();
   MX_REQUIRE(total_B == 0 || (B_offsets && vbe_row_output_offsets && vbe_b_t_map),
              "VBE needs B_offsets, row output offsets and the b_t map");
-  const Layout lay{total_B, B_offsets, vbe_row_output_offsets, vbe_b_t_map};
+  const Layout lay{total_B, B_offsets, vbe_row_output_offsets, vbe_b_t_map, 0};
   return backward_impl(weights, weights_ty, weights_offsets, D_offsets, T, max_B,
                        info_B_num_bits, lay, max_D, hash_size_cumsum, total_hash_size_bits,
                        indices, offsets, index_bytes, N, pooling_mode, indice_weights,
@@ -2309,55 +2393,18 @@ extern "C" int mx_tbe_backward_rowwise_adagrad_vbe(
 // Adagrad step of the pooled backward.  The nobag transpose's info of a
 // position is l * T + t (int64).
 //
-// Design: the batch is recast as a variable batch in which every position is
-// a bag of length one: bag l has offsets l and l + 1, belongs to table t with
-// b = l - offsets[t*B] (the b_t word (t << nb) | b), and its gradient row
-// starts at l * D.  The sort, run encoding and update then run unchanged.
-// Needs offsets[0] = 0 and offsets[T*B] = N, as upstream.
+// Design: every position is a bag of its own, the b-th of its table t's
+// positions (from offsets[t*B] on): its info word is (t << nb) | b and its
+// gradient row starts at l * D.  The sort, run encoding and update are the
+// pooled backward's; only linearize and the gradient row of an occurrence know
+// the difference, from the offsets themselves (arrays of the positions as bags,
+// built by a launch of their own and read by both, cost 7 us of a 96-column
+// step of 146 and 20 bytes per position).  Needs offsets[0] = 0 and offsets[T*B] = N,
+// as upstream.
 namespace mx {
 namespace {
 
-constexpr int kNobagMaxT = 1024;  // tables whose first positions fit LDS
-
-template <typename I>
-__global__ void __launch_bounds__(256)
-    nobag_layout_kernel(const I* __restrict__ offsets, int32_t T, int64_t B, int64_t N,
-                        int32_t D, int32_t nb, I* __restrict__ bag_offsets,
-                        int32_t* __restrict__ b_t_map, int64_t* __restrict__ row_out,
-                        int32_t* __restrict__ B_offsets, int32_t* __restrict__ D_offsets) {
-  __shared__ int64_t s_pos[kNobagMaxT + 1];
-  const bool lds = T <= kNobagMaxT;
-  if (lds)
-    for (int t = threadIdx.x; t <= T; t += 256) s_pos[t] = static_cast<int64_t>(offsets[t * B]);
-  __syncthreads();
-  if (blockIdx.x == 0) {
-    for (int t = threadIdx.x; t <= T; t += 256) {
-      if (B_offsets) B_offsets[t] = static_cast<int32_t>(offsets[t * B]);
-      if (D_offsets) D_offsets[t] = t * D;
-    }
-    if (threadIdx.x == 0) bag_offsets[N] = static_cast<I>(N);
-  }
-  for (int64_t l = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; l < N;
-       l += static_cast<int64_t>(gridDim.x) * 256) {
-    int32_t lo = 0, hi = T;  // pos[lo] <= l < pos[hi] (lo = 0 or T - 1 outside every bag)
-    while (hi - lo > 1) {
-      const int32_t mid = lo + ((hi - lo) >> 1);
-      const int64_t pm = lds ? s_pos[mid] : static_cast<int64_t>(offsets[mid * B]);
-      if (pm <= l)
-        lo = mid;
-      else
-        hi = mid;
-    }
-    const int64_t p = lds ? s_pos[lo] : static_cast<int64_t>(offsets[lo * B]);
-    const int64_t b = l - p > 0 ? l - p : 0;
-    bag_offsets[l] = static_cast<I>(l);
-    b_t_map[l] = static_cast<int32_t>((nb >= 32 ? 0u : (static_cast<uint32_t>(lo) << nb)) |
-                                      static_cast<uint32_t>(b));
-    if (row_out) row_out[l] = l * D;
-  }
-}
-
-// Sorted (t << nb) | b words of the recast batch -> the nobag infos l * T + t.
+// Sorted (t << nb) | b words -> the nobag infos l * T + t.
 template <typename I>
 __global__ void __launch_bounds__(256)
     nobag_infos_kernel(const int32_t* __restrict__ infos, const I* __restrict__ offsets,
@@ -2370,55 +2417,6 @@ __global__ void __launch_bounds__(256)
     const int64_t l = static_cast<int64_t>(offsets[t * B]) + static_cast<int64_t>(w & bmask);
     out[i] = l * T + t;
   }
-}
-
-// The recast batch's arrays, after the backward's (or transpose's) workspace.
-struct NobagWs {
-  void* bag_offsets;  // [N + 1] of the index type
-  int32_t* b_t_map;   // [N]
-  int64_t* row_out;   // [N]
-  int32_t* B_offsets; // [T + 1]
-  int32_t* D_offsets; // [T + 1]
-  int32_t* infos;     // [N] (transpose: the sorted b_t words)
-  size_t bytes;
-};
-
-NobagWs carve_nobag(uint8_t* base, size_t off, int64_t N, int32_t T, int32_t index_bytes) {
-  NobagWs w{};
-  auto take = [&](size_t bytes) {
-    uint8_t* p = base ? base + off : nullptr;
-    off += align256(bytes);
-    return p;
-  };
-  const int64_t n = N > 0 ? N : 1;
-  w.bag_offsets = take(static_cast<size_t>(n + 1) * static_cast<size_t>(index_bytes));
-  w.b_t_map = reinterpret_cast<int32_t*>(take(n * 4));
-  w.row_out = reinterpret_cast<int64_t*>(take(n * 8));
-  w.B_offsets = reinterpret_cast<int32_t*>(take(static_cast<size_t>(T + 1) * 4));
-  w.D_offsets = reinterpret_cast<int32_t*>(take(static_cast<size_t>(T + 1) * 4));
-  w.infos = reinterpret_cast<int32_t*>(take(n * 4));
-  w.bytes = off;
-  return w;
-}
-
-int launch_nobag_layout(const void* offsets, int32_t index_bytes, int32_t T, int64_t B,
-                        int64_t N, int32_t D, int32_t nb, const NobagWs& w, bool backward,
-                        hipStream_t s) {
-  const int64_t want = ceil_div(N, 256);
-  const int64_t cap = static_cast<int64_t>(num_cus()) * 8;
-  const dim3 gd(static_cast<uint32_t>(want < 1 ? 1 : (want < cap ? want : cap)));
-  if (index_bytes == 8)
-    nobag_layout_kernel<int64_t><<<gd, 256, 0, s>>>(
-        static_cast<const int64_t*>(offsets), T, B, N, D, nb,
-        static_cast<int64_t*>(w.bag_offsets), w.b_t_map, backward ? w.row_out : nullptr,
-        w.B_offsets, backward ? w.D_offsets : nullptr);
-  else
-    nobag_layout_kernel<int32_t><<<gd, 256, 0, s>>>(
-        static_cast<const int32_t*>(offsets), T, B, N, D, nb,
-        static_cast<int32_t*>(w.bag_offsets), w.b_t_map, backward ? w.row_out : nullptr,
-        w.B_offsets, backward ? w.D_offsets : nullptr);
-  MX_LAUNCH_CHECK();
-  return MX_OK;
 }
 
 int check_nobag(int32_t T, int64_t B, int32_t D, int32_t index_bytes, int64_t N) {
@@ -2436,9 +2434,9 @@ int check_nobag(int32_t T, int64_t B, int32_t D, int32_t index_bytes, int64_t N)
 
 extern "C" size_t mx_tbe_backward_nobag_workspace_bytes(int64_t N, int32_t T,
                                                         int32_t total_hash_size_bits, int32_t D) {
+  (void)T;
   (void)total_hash_size_bits;
-  const size_t base = carve_bwd(nullptr, N, D > 0 ? D : 1).bytes;
-  return carve_nobag(nullptr, base, N, T > 0 ? T : 0, 8).bytes;
+  return carve_bwd(nullptr, N, D > 0 ? D : 1).bytes;
 }
 
 extern "C" int mx_tbe_backward_rowwise_adagrad_nobag(
@@ -2455,26 +2453,21 @@ extern "C" int mx_tbe_backward_rowwise_adagrad_nobag(
   MX_REQUIRE(offsets && workspace, "null pointer argument");
   const int32_t nb = mx_tbe_info_B_num_bits(T, N);
   MX_REQUIRE(nb > 0, "T=%d and N=%lld do not fit a 32-bit info word", T, (long long)N);
-  const size_t base = carve_bwd(nullptr, N, D).bytes;
-  const NobagWs nw = carve_nobag(static_cast<uint8_t*>(workspace), base, N, T, index_bytes);
-  if (workspace_bytes < nw.bytes)
-    return set_error(MX_EWORKSPACE, "workspace of %zu bytes needed", nw.bytes);
-  auto* s = as_stream(stream);
-  if (int rc = launch_nobag_layout(offsets, index_bytes, T, B, N, D, nb, nw, true, s)) return rc;
-  const Layout lay{N, nw.B_offsets, nw.row_out, nw.b_t_map};
+  const Layout lay{N, nullptr, nullptr, nullptr, B};
   // total_D = T * D: every table is D wide (the full-width instances apply).
-  return backward_impl(weights, weights_ty, weights_offsets, nw.D_offsets, T, N, nb, lay, D,
-                       hash_size_cumsum, total_hash_size_bits, indices, nw.bag_offsets,
-                       index_bytes, N, MX_POOL_SUM, nullptr, grad_output,
-                       static_cast<int64_t>(T) * D, momentum1,
+  return backward_impl(weights, weights_ty, weights_offsets, nullptr, T, N, nb, lay, D,
+                       hash_size_cumsum, total_hash_size_bits, indices, offsets, index_bytes, N,
+                       MX_POOL_SUM, nullptr, grad_output, static_cast<int64_t>(T) * D, momentum1,
                        momentum1_offsets, learning_rate, eps, weight_decay, weight_decay_mode,
-                       stochastic_rounding, rng, workspace, base, stream);
+                       stochastic_rounding, rng, workspace, workspace_bytes, stream);
 }
 
 extern "C" size_t mx_tbe_transpose_nobag_workspace_bytes(int64_t N, int32_t T,
                                                          int32_t total_hash_size_bits) {
+  (void)T;
   (void)total_hash_size_bits;
-  return carve_nobag(nullptr, carve_sort(nullptr, N).bytes, N, T > 0 ? T : 0, 8).bytes;
+  // The sort's workspace, then the sorted (t << nb) | b words.
+  return carve_sort(nullptr, N).bytes + align256(static_cast<size_t>(N > 0 ? N : 1) * 4);
 }
 
 extern "C" int mx_tbe_transpose_embedding_input_nobag(
@@ -2487,7 +2480,7 @@ extern "C" int mx_tbe_transpose_embedding_input_nobag(
   MX_REQUIRE(T >= 0 && B >= 0 && N >= 0, "negative T, B or N");
   MX_REQUIRE(index_bytes == 4 || index_bytes == 8, "indices must be int32 or int64");
   MX_REQUIRE(N < 0x7fffffffll, "N %lld too large for int32 positions", (long long)N);
-  const Layout empty{0, nullptr, nullptr, nullptr};
+  const Layout empty{0, nullptr, nullptr, nullptr, 0};
   if (N == 0)
     return transpose_impl(hash_size_cumsum, T, 0, empty, total_hash_size_bits, 26, indices,
                           offsets, index_bytes, 0, linear_indices, sorted_linear_indices,
@@ -2499,26 +2492,25 @@ extern "C" int mx_tbe_transpose_embedding_input_nobag(
   const int32_t nb = mx_tbe_info_B_num_bits(T, N);
   MX_REQUIRE(nb > 0, "T=%d and N=%lld do not fit a 32-bit info word", T, (long long)N);
   const size_t base = carve_sort(nullptr, N).bytes;
-  const NobagWs nw = carve_nobag(static_cast<uint8_t*>(workspace), base, N, T, index_bytes);
-  if (workspace_bytes < nw.bytes)
-    return set_error(MX_EWORKSPACE, "workspace of %zu bytes needed", nw.bytes);
+  const size_t need = mx_tbe_transpose_nobag_workspace_bytes(N, T, total_hash_size_bits);
+  if (workspace_bytes < need)
+    return set_error(MX_EWORKSPACE, "workspace of %zu bytes needed", need);
+  auto* words = reinterpret_cast<int32_t*>(static_cast<uint8_t*>(workspace) + base);
   auto* s = as_stream(stream);
-  if (int rc = launch_nobag_layout(offsets, index_bytes, T, B, N, 4, nb, nw, false, s)) return rc;
-  const Layout lay{N, nw.B_offsets, nullptr, nw.b_t_map};  // B_offsets: per-feature sort segments
+  const Layout lay{N, nullptr, nullptr, nullptr, B};
   if (int rc = transpose_impl(hash_size_cumsum, T, 0, lay, total_hash_size_bits, nb, indices,
-                              nw.bag_offsets, index_bytes, N, linear_indices,
-                              sorted_linear_indices, nw.infos, sorted_linear_indices_run,
-                              run_lengths, num_runs, cumulative_run_lengths, workspace, base,
-                              stream))
+                              offsets, index_bytes, N, linear_indices, sorted_linear_indices,
+                              words, sorted_linear_indices_run, run_lengths, num_runs,
+                              cumulative_run_lengths, workspace, base, stream))
     return rc;
   const int64_t want = ceil_div(N, 256);
   const int64_t cap = static_cast<int64_t>(num_cus()) * 8;
   const dim3 gd(static_cast<uint32_t>(want < cap ? want : cap));
   if (index_bytes == 8)
-    nobag_infos_kernel<int64_t><<<gd, 256, 0, s>>>(nw.infos, static_cast<const int64_t*>(offsets),
+    nobag_infos_kernel<int64_t><<<gd, 256, 0, s>>>(words, static_cast<const int64_t*>(offsets),
                                                    T, B, N, nb, infos_sorted);
   else
-    nobag_infos_kernel<int32_t><<<gd, 256, 0, s>>>(nw.infos, static_cast<const int32_t*>(offsets),
+    nobag_infos_kernel<int32_t><<<gd, 256, 0, s>>>(words, static_cast<const int32_t*>(offsets),
                                                    T, B, N, nb, infos_sorted);
   MX_LAUNCH_CHECK();
   return MX_OK;
