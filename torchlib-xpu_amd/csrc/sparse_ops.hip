@@ -406,6 +406,9 @@ __device__ __forceinline__ void perm_copy(const E* __restrict__ in, E* __restric
         for (int v = 0; v < V; ++v) x[k][v] = o + v < o1 ? in[o + v + shift] : E(0);
       }
     }
+    // Once, and not again before each store behind the store before it (100
+    // features of 8192 bags 110.7 -> 101.0 us, 40 of 4096 26.9 -> 26.3).
+    wait_loads();
 #pragma unroll
     for (int k = 0; k < K; ++k) {
       const int64_t o = base + (k * kPermThreads + static_cast<int64_t>(threadIdx.x)) * V;
