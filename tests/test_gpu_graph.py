@@ -256,8 +256,7 @@ def test_fp16_stochastic_rounding_graph_replays_draw_fresh_bits(dev):
 
 
 def test_nobag_training_step_graph_replays_match_eager(dev):
-    """PoolingMode NONE: the nobag forward, the nobag backward (its batch recast
-    as one-position bags on the device) and an nbit nobag lookup, captured
+    """PoolingMode NONE: the nobag forward, the nobag backward and an nbit nobag lookup, captured
     together; every replay equals the eager step bit for bit."""
     print("[case] graph-captured nobag forward + backward + nbit nobag, 4 replays", flush=True)
     rng = np.random.default_rng(6)

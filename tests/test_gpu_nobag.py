@@ -346,7 +346,7 @@ def test_inference_module_nobag(dev, out):
 
 @pytest.mark.parametrize("layout", ["empty_first", "empty_middle", "empty_last", "shared_table"])
 def test_nobag_sort_segments(dev, layout):
-    """The recast batch sorts in per-feature segments: whole features without
+    """A sequence batch sorts in per-feature segments: whole features without
     positions (first, middle, last) and two features sharing one table (equal
     hash_size_cumsum entries: one segment), each feature over several
     3072-key sort tiles; backward and transpose against the oracle."""

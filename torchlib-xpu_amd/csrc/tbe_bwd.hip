@@ -2066,7 +2066,7 @@ int launch_bwd(const BwdArgs& a, SortWs& ws, uint32_t* chunk_start, int64_t N, h
 
 // Full-width instance when every table's D equals the row width of the
 // chosen (G, NCH): total_D = T * max_D says so (no D exceeds max_D, and the
-// D_offsets sum to total_D: a fixed batch's grad_output width, the recast
+// D_offsets sum to total_D: a fixed batch's grad_output width, a
 // sequence batch's T * D; a variable batch passes 0).  Plain instance for SUM
 // pooling without weights or weight decay.
 template <typename I, typename WT, int G, int NCH>
