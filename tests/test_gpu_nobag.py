@@ -405,3 +405,49 @@ def test_nobag_sort_segments(dev, layout):
     np.testing.assert_array_equal(run[:r], exp["run"])
     np.testing.assert_array_equal(lens[:r], exp["run_lengths"])
     np.testing.assert_array_equal(cum[:r + 1], exp["cumulative_run_lengths"])
+
+
+@pytest.mark.parametrize("N", [3000, 12000])
+@pytest.mark.parametrize("layout", ["head", "tail", "all", "overlap"])
+def test_nobag_positions_outside_bags(dev, N, layout):
+    """Positions before the first bag count as table 0's and positions past the
+    last as the last table's, each with its own gradient row (all: no bag holds
+    any position, every offset is N), either side of 8192 positions.  In
+    `overlap` table 1 (the rows of table 0, one sort segment) ends before it
+    starts: the segments do not hold the positions of their tables, so the
+    batch sorts as one."""
+    print(f"[case] nobag outside bags N={N} {layout}", flush=True)
+    rng = np.random.default_rng(N)
+    T, B, D = 3, 4, 36
+    hsc = np.array([0, 0, 50, 120], np.int64)
+    q = N // 4
+    first = {"head": [q, 2 * q, 3 * q, N], "tail": [0, q, 2 * q, 3 * q], "all": [N] * 4,
+             "overlap": [0, 2 * q, q, N]}[layout]
+    seen = {"head": [0, 2 * q, 3 * q, N], "tail": [0, q, 2 * q, N], "all": [0, N, N, N],
+            "overlap": [0, 2 * q, 2 * q, N]}[layout]
+    offsets, covering = (np.repeat(np.asarray(f, np.int64), B)[:T * B + 1] for f in (first, seen))
+    rows = np.where(np.arange(N) < seen[2], 50, 70)
+    indices = rng.integers(0, rows)
+    w_off, m1_off, bits = hsc[:-1] * D, hsc[:-1].copy(), 7
+    W = rng.uniform(-0.5, 0.5, size=120 * D).astype(np.float32)
+    m1 = rng.uniform(0, 0.01, size=120).astype(np.float32)
+    grad = rng.normal(0, 0.01, size=(N, D)).astype(np.float32)
+    Wd, m1d = torch.from_numpy(W).to(dev), torch.from_numpy(m1).to(dev)
+    empty = torch.zeros(0, device=dev)
+    pl = torch.zeros(T, dtype=torch.int32, device=dev)
+    hsc_d = torch.from_numpy(hsc).to(dev)
+    idx_d, off_d = torch.from_numpy(indices).to(dev), torch.from_numpy(offsets).to(dev)
+    out = torch.ops.fbgemm.transpose_embedding_input(hsc_d, bits, idx_d, off_d, True)
+    exp = orc.transpose_embedding_input_nobag(hsc, B, bits, indices, covering)
+    assert int(out[5].item()) == exp["num_runs"]
+    np.testing.assert_array_equal(out[1].cpu().numpy(), exp["sorted_linear_indices"])
+    np.testing.assert_array_equal(out[2].cpu().numpy(), exp["infos_sorted"])
+    torch.ops.fbgemm.split_embedding_nobag_backward_codegen_rowwise_adagrad_unweighted_exact_cuda(
+        torch.from_numpy(grad).to(dev), Wd, empty, empty, pl, torch.from_numpy(w_off).to(dev),
+        D, hsc_d, bits, idx_d, off_d, torch.zeros(0, dtype=torch.int32, device=dev), 0, 0,
+        False, m1d, empty, pl, torch.from_numpy(m1_off).to(dev), 1e-8, 0.05, 0.0, 0, 0.0)
+    W_exp, m_exp = orc.backward_rowwise_adagrad_nobag(
+        W, w_off, D, B, hsc, bits, indices, covering, grad, m1, m1_off, 0.05, 1e-8)
+    # Long runs sum in 32-row chunks: the bounds of the duplicate-heavy cases above.
+    np.testing.assert_allclose(m1d.cpu().numpy(), m_exp, rtol=1e-4, atol=0)
+    np.testing.assert_allclose(Wd.cpu().numpy(), W_exp, rtol=RTOL, atol=1e-6)

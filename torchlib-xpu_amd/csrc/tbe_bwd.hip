@@ -158,9 +158,17 @@ __device__ __forceinline__ int32_t seq_table(int64_t l, int32_t T, First first) 
   return lo;
 }
 
+// First position of a sequence batch's table t.  Positions before offsets[0] lie
+// in no bag and count as table 0's, so first + (place in the table) is a
+// position's own number, which its gradient row goes by, whatever the offsets.
+template <typename I>
+__device__ __forceinline__ int64_t seq_first(const I* offsets, int64_t t, int64_t seq_B) {
+  return t == 0 ? 0 : static_cast<int64_t>(offsets[t * seq_B]);
+}
+
 // SEQ: a sequence batch, in which every position is a bag of its own: table t's
-// positions start at offsets[t * seq_B], a position's info word holds t and its
-// place among them, and no bag is searched.
+// positions start at offsets[t * seq_B] (seq_first), a position's info word holds
+// t and its place among them, and no bag is searched.
 template <typename I, bool SEQ>
 __global__ void __launch_bounds__(256)
     linearize_kernel(const int64_t* __restrict__ hsc, const I* __restrict__ indices,
@@ -188,7 +196,7 @@ __global__ void __launch_bounds__(256)
   __shared__ int64_t s_first[SEQ ? kNobagMaxT + 1 : 1];  // first position of each table
   const bool first_lds = T <= kNobagMaxT;
   auto first = [&](int64_t t) -> int64_t {
-    return SEQ && first_lds ? s_first[t] : static_cast<int64_t>(offsets[t * seq_B]);
+    return SEQ && first_lds ? s_first[t] : seq_first(offsets, t, seq_B);
   };
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int64_t l0 = static_cast<int64_t>(blockIdx.x) * kLinTile;
@@ -210,7 +218,7 @@ __global__ void __launch_bounds__(256)
   const int32_t lane_boff = seg.B_off && w == 0 && lane <= seg.T ? seg.B_off[lane] : 0;
   if constexpr (SEQ) {
     if (first_lds)
-      for (int t = threadIdx.x; t <= T; t += 256) s_first[t] = static_cast<int64_t>(offsets[t * seq_B]);
+      for (int t = threadIdx.x; t <= T; t += 256) s_first[t] = seq_first(offsets, t, seq_B);
     if (threadIdx.x < 2) s_range[threadIdx.x][0] = 0;
     __syncthreads();
   }
@@ -375,8 +383,7 @@ __global__ void __launch_bounds__(256)
       int64_t t;
       if constexpr (SEQ) {
         t = rel[it];
-        const int64_t b = l - first(t) > 0 ? l - first(t) : 0;
-        info = (nb >= 32 ? 0u : (rel[it] << nb)) | static_cast<uint32_t>(b);
+        info = (nb >= 32 ? 0u : (rel[it] << nb)) | static_cast<uint32_t>(l - first(t));
       } else if (b_t_map) {
         info = static_cast<uint32_t>(b_t_map[bag]);
         t = nb >= 32 ? 0 : static_cast<int64_t>(info >> nb);
@@ -447,6 +454,9 @@ __global__ void __launch_bounds__(256)
         const uint32_t incl = wave_incl_scan<SumOp>(nt);
         // The segments must also cover exactly the positions [0, N).
         bool bad = (lane < S && fnext < fp) || (lane == 0 && fp != 0) || (lane == S && fp != N);
+        // A sequence batch's positions find their tables by the first positions of
+        // all of them, also of those that share a segment.
+        if constexpr (SEQ) bad = bad || (lane < T && first(lane + 1) < first(lane));
         if (lane <= T) seg.fpos[lane] = fp;
         if (lane < T) seg.tprefix[lane + 1] = static_cast<int32_t>(incl);
         if (lane == 0) seg.tprefix[0] = 0;
@@ -1013,11 +1023,12 @@ __global__ void __launch_bounds__(kSweepThreads) small_transpose_kernel(SmallSor
       uint32_t info;
       int64_t t;
       if (a.seq_B) {
-        auto first = [&](int64_t x) { return static_cast<int64_t>(offsets[x * a.seq_B]); };
-        const int32_t ts = seq_table(i, a.T, first);
-        const int64_t b = i - first(ts) > 0 ? i - first(ts) : 0;
+        // The search probes tables from 1 on, whose first positions are the offsets'.
+        const int32_t ts = seq_table(
+            i, a.T, [&](int64_t x) { return static_cast<int64_t>(offsets[x * a.seq_B]); });
         t = ts;
-        info = (a.nb >= 32 ? 0u : (static_cast<uint32_t>(ts) << a.nb)) | static_cast<uint32_t>(b);
+        info = (a.nb >= 32 ? 0u : (static_cast<uint32_t>(ts) << a.nb)) |
+               static_cast<uint32_t>(i - seq_first(offsets, t, a.seq_B));
       } else if (a.b_t_map) {
         info = static_cast<uint32_t>(a.b_t_map[bag]);
         t = a.nb >= 32 ? 0 : static_cast<int64_t>(info >> a.nb);
@@ -1500,7 +1511,7 @@ struct BwdArgs {
   const float* iw_sorted;  // per-sample weights in sorted order, or null
   const int32_t* B_off;    // VBE: first bag of each table [T+1], or null (fixed batch)
   const int64_t* row_out;  // VBE: gradient row offset of each bag, or null
-  int64_t seq_B;           // sequence batch: position offsets[t * seq_B] + b has row * max_D; else 0
+  int64_t seq_B;           // sequence batch: position seq_first(t) + b has row * max_D; else 0
   const uint32_t* num_runs;
   const uint32_t* chunk_start;
   const uint32_t* chunk_mark;  // chunk marks (kMarkEvery), from the chunk-count scan
@@ -1671,7 +1682,7 @@ __device__ void group_sum_occurrences(const BwdArgs& a, const MetaView& mv, int3
       // Full width: every feature's columns start at tj * G*NCH*4 (config 3:
       // chunk sums 14.5 -> 12.8 us against the table lookup).
       if (a.seq_B)
-        my_row = (static_cast<int64_t>(static_cast<const I*>(a.offsets)[tj * a.seq_B]) + b) * a.max_D;
+        my_row = (seq_first(static_cast<const I*>(a.offsets), tj, a.seq_B) + b) * a.max_D;
       else
         my_row = a.row_out ? a.row_out[bag]
                            : b * a.total_D + (FULL ? tj * (G * NCH * 4) : mv.D_off(tj));
@@ -2399,8 +2410,9 @@ extern "C" int mx_tbe_backward_rowwise_adagrad_vbe(
 // pooled backward's; only linearize and the gradient row of an occurrence know
 // the difference, from the offsets themselves (arrays of the positions as bags,
 // built by a launch of their own and read by both, cost 7 us of a 96-column
-// step of 146 and 20 bytes per position).  Needs offsets[0] = 0 and offsets[T*B] = N,
-// as upstream.
+// step of 146 and 20 bytes per position).  Upstream needs offsets[0] = 0 and
+// offsets[T*B] = N; here positions before the first bag go with table 0 and
+// positions past the last with table T - 1, each with its own gradient row.
 namespace mx {
 namespace {
 
@@ -2414,7 +2426,7 @@ __global__ void __launch_bounds__(256)
        i += static_cast<int64_t>(gridDim.x) * 256) {
     const uint32_t w = static_cast<uint32_t>(infos[i]);
     const int64_t t = nb >= 32 ? 0 : static_cast<int64_t>(w >> nb);
-    const int64_t l = static_cast<int64_t>(offsets[t * B]) + static_cast<int64_t>(w & bmask);
+    const int64_t l = seq_first(offsets, t, B) + static_cast<int64_t>(w & bmask);
     out[i] = l * T + t;
   }
 }
