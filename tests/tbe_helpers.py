@@ -21,6 +21,29 @@ def random_tbe(rng: np.random.Generator, T: int, B: int, dims, rows, max_L: int,
     return bench_inputs.TbeInput(T=T, E=list(rows), D=list(dims), B=B, indices=idx, offsets=off)
 
 
+def gpu_us(fn, calls: int = 20, rounds: int = 5) -> float:
+    """Device time of one call of `fn`, microseconds: the best of a few rounds of
+    calls captured as one graph (what the host takes to submit them is left out)."""
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        fn()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        for _ in range(calls):
+            fn()
+    best = float("inf")
+    for _ in range(rounds + 1):
+        start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        start.record()
+        graph.replay()
+        end.record()
+        torch.cuda.synchronize()
+        best = min(best, start.elapsed_time(end) * 1e3 / calls)
+    return best
+
+
 def weight_offsets(inp: bench_inputs.TbeInput) -> np.ndarray:
     sizes = [E * D for E, D in zip(inp.E, inp.D)]
     return np.concatenate([[0], np.cumsum(sizes)[:-1]]).astype(np.int64)

@@ -7,6 +7,7 @@ import torch
 
 import oracle as orc
 from mx_fbgemm import bench_inputs
+from tbe_helpers import gpu_us
 
 pytestmark = pytest.mark.gpu
 
@@ -112,6 +113,82 @@ def test_bag_group_sizes(dev, dims, max_L, D):
     added, _ = torch.ops.fbgemm.jagged_dense_elementwise_add_jagged_output(
         torch.from_numpy(vals).to(dev), ot, torch.from_numpy(dense).to(dev))
     _bits_equal(added, orc.jagged_dense_elementwise_add(vals, offs, dense, "f32"))
+
+
+@pytest.mark.parametrize("dims", [1, 2, 3])
+@pytest.mark.parametrize("head,tail", [(0, 0), (700, 0), (0, 900), (40, 30000)])
+@pytest.mark.parametrize("longest,max_L,D,dt", [(50, 4, 4, "f32"), (3000, 40, 16, "f32"),
+                                                (40000, 3, 5, "bf16"), (2000, 2500, 64, "bf16")])
+def test_lists_past_their_cap(dev, dims, head, tail, longest, max_L, D, dt):
+    """One list among 600 short ones, up to thousands of times as long: its rows
+    past what its group takes (more than eight usual lists, cut by max_length or
+    not) and the rows before the first list and past the last come from row
+    windows of the grid, at 1 to 3 jagged dims; below and above the size at which
+    a group takes any list whole.  Copy and add bit-exact."""
+    print(f"[case] jagged cap dims={dims} longest={longest} max_L={max_L} D={D} head={head} "
+          f"tail={tail} {dt}", flush=True)
+    rng = np.random.default_rng(longest + dims)
+    lengths = rng.integers(0, 5, 600)
+    lengths[[0, 333, 599][dims - 1]] = longest
+    outer = {1: [], 2: [[150] * 4], 3: [[2, 0, 2], [200, 50, 250, 100]]}[dims]
+    maxs = {1: [], 2: [140], 3: [2, 250]}[dims] + [max_L]
+    offs = [_offsets(o) for o in outer] + [_offsets(lengths) + head]
+    n = int(offs[-1][-1]) + tail
+    B = offs[0].size - 1
+    tdt = torch.float32 if dt == "f32" else torch.bfloat16
+    vals = torch.from_numpy(rng.standard_normal((n, D)).astype(np.float32)).to(tdt)
+    dense = torch.from_numpy(rng.standard_normal((B, *maxs, D)).astype(np.float32)).to(tdt)
+    ot = [torch.from_numpy(o).to(dev) for o in offs]
+    # Expected by place: row l of list p is dense[coordinates of p, l - off[p]].
+    exp = torch.zeros((n, D), dtype=tdt)
+    for p in range(600):
+        path, q = [], p
+        for o in reversed(offs[:-1]):
+            parent = int(np.searchsorted(o, q, side="right")) - 1
+            path.insert(0, q - int(o[parent]))
+            q = parent
+        if any(c >= m for c, m in zip(path, maxs)):
+            continue
+        b, e = int(offs[-1][p]), int(offs[-1][p + 1])
+        e = min(e, b + max_L)
+        exp[b:e] = dense[(q, *path)][: e - b]
+    back, _ = torch.ops.fbgemm.dense_to_jagged(dense.to(dev), ot, n)
+    assert torch.equal(back.cpu().view(torch.uint8), exp.view(torch.uint8))
+    added, _ = torch.ops.fbgemm.jagged_dense_elementwise_add_jagged_output(
+        vals.to(dev), ot, dense.to(dev))
+    want = (vals.float() + exp.float()).to(tdt)  # one rounding per element
+    assert torch.equal(added.cpu().view(torch.uint8), want.view(torch.uint8))
+
+
+@pytest.mark.parametrize("dims", [1, 2])
+@pytest.mark.parametrize("op", ["copy", "add"])
+def test_one_long_list_is_spread(dev, dims, op):
+    """A batch whose rows nearly all lie in one list, or in none, takes at most ten
+    times an even batch of the same rows (served by one group of threads: a
+    hundred to a thousand times)."""
+    print(f"[case] jagged one long list dims={dims} {op}", flush=True)
+    n, L, D = 2048, 100, 16
+    total = n * L
+
+    def call(lengths, extra=0):
+        offs = ([_offsets([32] * (n // 32))] if dims == 2 else []) + [_offsets(lengths)]
+        maxs = [32, L] if dims == 2 else [L]
+        ot = [torch.from_numpy(o).to(dev) for o in offs]
+        dense = torch.randn(offs[0].size - 1, *maxs, D, device=dev)
+        vals = torch.randn(int(offs[-1][-1]), D, device=dev)
+        if op == "copy":
+            return gpu_us(lambda: torch.ops.fbgemm.dense_to_jagged(
+                dense, ot, int(offs[-1][-1]) + extra))
+        return gpu_us(lambda: torch.ops.fbgemm.jagged_dense_elementwise_add_jagged_output(
+            vals, ot, dense))
+
+    even = call([L] * n)
+    skewed = np.full(n, 1)
+    skewed[n // 3] = total - n + 1
+    one = call(skewed)
+    none = call([1] * n, total - n) if op == "copy" else 0.0
+    print(f"even {even:.1f} us, one list {one:.1f}, no list {none:.1f}", flush=True)
+    assert one <= 10 * even and none <= 10 * even
 
 
 def test_two_jagged_dims(dev):

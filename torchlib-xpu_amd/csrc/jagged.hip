@@ -19,6 +19,8 @@
 // 64 or 256 threads by the bag's size.  (Two jagged dims, 256 x 20 x 50 x 64
 // bf16, against coordinates per chunk: padding 26.6 -> 11.3 us, back 14.3 ->
 // 11.0 by trace; the fp32 add 21.2 -> 15.6 us per call.)
+#include <type_traits>
+
 #include "mx_common.h"
 
 namespace mx {
@@ -35,6 +37,15 @@ template <int VEC>
 struct alignas(VEC) Chunk {
   uint8_t b[VEC];
 };
+
+// In whole words: cleared byte by byte, a chunk that may also be loaded lives in a
+// register per byte, and its load is waited for at once.
+template <int VEC>
+__device__ __forceinline__ void clear(Chunk<VEC>& c) {
+  using W = std::conditional_t<(VEC >= 4), uint32_t, std::conditional_t<VEC == 2, uint16_t, uint8_t>>;
+#pragma unroll
+  for (int e = 0; e < VEC; e += static_cast<int>(sizeof(W))) *reinterpret_cast<W*>(c.b + e) = W(0);
+}
 
 template <typename I>
 __device__ __forceinline__ int64_t off_at(const JaggedMeta& m, int k, int64_t i) {
@@ -110,10 +121,9 @@ __device__ __forceinline__ float bf16_to_f32(uint16_t h) {
 }
 // Round to nearest even, NaN kept quiet (same rule as c10::BFloat16).
 __device__ __forceinline__ uint16_t f32_to_bf16(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return static_cast<uint16_t>((u >> 16) | 0x40);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return static_cast<uint16_t>(u >> 16);
+  const uint32_t u = __float_as_uint(f);
+  const uint32_t r = (u + 0x7fffu + ((u >> 16) & 1u)) >> 16, nan = (u >> 16) | 0x40u;
+  return static_cast<uint16_t>((u & 0x7fffffffu) > 0x7f800000u ? nan : r);
 }
 
 // x (op) y per element in the element type's arithmetic: f32/f64 natively,
@@ -154,6 +164,17 @@ struct BinOp<MX_DTYPE_BF16, MUL> {
     const float a = bf16_to_f32(*reinterpret_cast<const uint16_t*>(x));
     const float b = bf16_to_f32(*reinterpret_cast<const uint16_t*>(y));
     *reinterpret_cast<uint16_t*>(o) = f32_to_bf16(MUL ? a * b : a + b);
+  }
+  // Two elements of one 32-bit word.  The asm holds the unpacking back to here:
+  // else the compiler unpacks every word as it is loaded, into twice the
+  // registers (150 in all, three waves per SIMD).
+  __device__ static void apply_word(const uint8_t* x, const uint8_t* y, uint8_t* o) {
+    uint32_t a = *reinterpret_cast<const uint32_t*>(x), b = *reinterpret_cast<const uint32_t*>(y);
+    asm("" : "+v"(a), "+v"(b));
+    const float a0 = __uint_as_float(a << 16), a1 = __uint_as_float(a & 0xffff0000u);
+    const float b0 = __uint_as_float(b << 16), b1 = __uint_as_float(b & 0xffff0000u);
+    *reinterpret_cast<uint32_t*>(o) = f32_to_bf16(MUL ? a0 * b0 : a0 + b0) |
+                                      (static_cast<uint32_t>(f32_to_bf16(MUL ? a1 * b1 : a1 + b1)) << 16);
   }
 };
 
@@ -219,44 +240,47 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// Values rows [r0, r1) whose first `copy_rows` rows take dense rows from
-// `dense_row0` on and the rest 0; ADD combines x with them (x + y, or x * y
-// with MUL), else the dense value is copied (dense -> jagged).
+// Part `part` of `parts` of values rows [r0, r1), whose first `copy_rows` rows
+// take dense rows from `dense_row0` on and the rest 0; ADD combines x with them
+// (x + y, or x * y with MUL), else the dense value is copied (dense -> jagged).
 template <int VEC, bool ADD, int DT, bool MUL>
 __device__ __forceinline__ void emit_rows(const uint8_t* __restrict__ dense,
                                           const uint8_t* __restrict__ x,
                                           uint8_t* __restrict__ out, int64_t r0, int64_t r1,
                                           int64_t copy_rows, int64_t dense_row0, int64_t vpr,
-                                          int32_t tpb) {
+                                          int32_t tpb, int64_t part, int64_t parts) {
   const int32_t t = threadIdx.x & (tpb - 1);
   const int64_t span = static_cast<int64_t>(tpb) * kJagItems;
   const int64_t n_all = (r1 - r0) * vpr, n_copy = copy_rows * vpr;
   const Chunk<VEC>* __restrict__ src = reinterpret_cast<const Chunk<VEC>*>(dense) + dense_row0 * vpr;
   Chunk<VEC>* __restrict__ dst = reinterpret_cast<Chunk<VEC>*>(out) + r0 * vpr;
   const Chunk<VEC>* __restrict__ xs = reinterpret_cast<const Chunk<VEC>*>(x) + r0 * vpr;
-  for (int64_t base = blockIdx.y * span; base < n_all; base += gridDim.y * span) {
+  for (int64_t base = part * span; base < n_all; base += parts * span) {
     Chunk<VEC> y[kJagItems];
+    [[maybe_unused]] Chunk<VEC> cx[kJagItems];
 #pragma unroll
     for (int it = 0; it < kJagItems; ++it) {
       const int64_t i = base + it * tpb + t;
-      if (i < n_copy) {
-        y[it] = src[i];
-      } else {
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) y[it].b[e] = 0;  // +0 in every element type
-      }
+      if constexpr (ADD)
+        if (i < n_all) cx[it] = xs[i];
+      if (i < n_copy) y[it] = src[i];
     }
-    if constexpr (!ADD) wait_loads();
+    wait_loads();
 #pragma unroll
     for (int it = 0; it < kJagItems; ++it) {
       const int64_t i = base + it * tpb + t;
       if (i >= n_all) continue;
+      if (i >= n_copy) clear(y[it]);  // +0 in every element type
       if constexpr (ADD) {
-        const Chunk<VEC> cx = xs[i];
+        using Op = BinOp<DT, MUL>;
         Chunk<VEC> co;
+        if constexpr (DT == MX_DTYPE_BF16 && VEC >= 4) {
 #pragma unroll
-        for (int e = 0; e < VEC; e += BinOp<DT, MUL>::kBytes)
-          BinOp<DT, MUL>::apply(cx.b + e, y[it].b + e, co.b + e);
+          for (int e = 0; e < VEC; e += 4) Op::apply_word(cx[it].b + e, y[it].b + e, co.b + e);
+        } else {
+#pragma unroll
+          for (int e = 0; e < VEC; e += Op::kBytes) Op::apply(cx[it].b + e, y[it].b + e, co.b + e);
+        }
         dst[i] = co;
       } else {
         dst[i] = y[it];
@@ -265,62 +289,149 @@ __device__ __forceinline__ void emit_rows(const uint8_t* __restrict__ dense,
   }
 }
 
-// Group x < nlists: innermost list x.  Group x == nlists: the values rows no
-// list covers (before the first offset, from the last on), which have no dense
-// position.  Row ranges are clamped to [0, total_L], so malformed offsets never
-// write out of bounds.
+// How the values rows are dealt out.  The groups of the first list_blocks
+// columns of the grid take the innermost lists, each its first cap rows; what a
+// longer list holds past them, and the rows that no list covers, fall to windows
+// of `window` rows (at most cap), a block each, in the columns after.  So a list
+// far longer than the others -- or than max_length, past which rows are only
+// cleared -- is spread over the grid.  (512 lists of 8 rows but one of 200,000, 16
+// fp32 columns, max_length 16: 2,950 us with each list to one group, 7.4; the add
+// 18,200 and 8.7; 500,000 rows past the last list, two jagged dims, 64 columns:
+// 1,776 and 32.  A batch without either pays for windows that find nothing: 300
+// lists of 20 rows 2.6 us, 2.7.)
+struct ListGrid {
+  int64_t list_blocks;
+  int64_t cap;
+  int64_t window;
+  int64_t windows;
+};
+
+// The list that row x lies in: the last p in [0, n) with off[p] <= x (0 if none).
+// A wave's lanes probe 64 offsets per round.
+template <typename I>
+__device__ __forceinline__ int64_t wave_owner(const JaggedMeta& m, int k, int64_t n, int64_t x) {
+  const int lane = threadIdx.x & 63;
+  int64_t lo = 0, hi = n;
+  while (hi - lo > 1) {  // wave-uniform; the range shrinks whatever the offsets hold
+    const int64_t stride = (hi - lo + 63) >> 6, pos = lo + lane * stride;
+    const int c = __popcll(__ballot(off_at<I>(m, k, pos < hi ? pos : lo) <= x && pos < hi));
+    lo += (c > 0 ? c - 1 : 0) * stride;
+    hi = lo + stride < hi ? lo + stride : hi;
+  }
+  return lo;
+}
+
+// Row ranges are clamped to [0, total_L], so malformed offsets never write out
+// of bounds.
 template <int VEC, typename I, bool ADD, int DT, bool MUL, bool ONE>
 __global__ void __launch_bounds__(256)
     jagged_out_kernel(const uint8_t* __restrict__ dense, const uint8_t* __restrict__ x,
-                      uint8_t* __restrict__ out, JaggedMeta m, int64_t nlists, int32_t lg,
-                      int64_t total_L, int64_t vpr) {
-  if constexpr (ONE) {
-    lg = 8;
-    m.ndim = 1;
-  }
+                      uint8_t* __restrict__ out, const JaggedMeta m, int64_t nlists,
+                      int32_t group_lg, int64_t total_L, int64_t vpr, const ListGrid g) {
+  const int32_t lg = ONE ? 8 : group_lg;
   auto clamp = [&](int64_t v, int64_t lo) { return v < lo ? lo : (v > total_L ? total_L : v); };
-  const int last = m.ndim - 1;
+  const int last = ONE ? 0 : m.ndim - 1;
   const int64_t max_L = m.max_len[last];
-  const int32_t tpb = 1 << lg;
-  const int64_t step = static_cast<int64_t>(gridDim.x) << (8 - lg);
-  for (int64_t p = (static_cast<int64_t>(blockIdx.x) << (8 - lg)) + (threadIdx.x >> lg);
-       p <= nlists; p += step) {
-    if (p < nlists) {
+  // Of rows [s, e) of list p, whose rows are [r0, r1): how many have a dense row,
+  // and the first one's.
+  auto place = [&](int64_t p, int64_t r0, int64_t r1, int64_t s, int64_t e, int64_t& row) {
+    const int64_t bag = ONE ? p : list_dense_bag<I>(p, m);
+    const int64_t left = bag < 0 ? 0 : r0 + (r1 - r0 < max_L ? r1 - r0 : max_L) - s;
+    const int64_t copy = left < 0 ? 0 : (left < e - s ? left : e - s);
+    row = copy > 0 ? bag * max_L + (s - r0) : 0;
+    return copy;
+  };
+  if (static_cast<int64_t>(blockIdx.x) < g.list_blocks) {  // block-uniform
+    const int64_t step = g.list_blocks << (8 - lg);
+    for (int64_t p = (static_cast<int64_t>(blockIdx.x) << (8 - lg)) + (threadIdx.x >> lg);
+         p < nlists; p += step) {
       const int64_t r0 = clamp(off_at<I>(m, last, p), 0);
       const int64_t r1 = clamp(off_at<I>(m, last, p + 1), r0);
       if (r1 == r0) continue;
-      const int64_t bag = list_dense_bag<I>(p, m);
-      const int64_t copy = bag < 0 ? 0 : (r1 - r0 < max_L ? r1 - r0 : max_L);
-      emit_rows<VEC, ADD, DT, MUL>(dense, x, out, r0, r1, copy, bag < 0 ? 0 : bag * max_L, vpr,
-                                   tpb);
-    } else {
-      const int64_t head = clamp(off_at<I>(m, last, 0), 0);
-      const int64_t tail = clamp(off_at<I>(m, last, nlists), head);
-      emit_rows<VEC, ADD, DT, MUL>(dense, x, out, 0, head, 0, 0, vpr, tpb);
-      emit_rows<VEC, ADD, DT, MUL>(dense, x, out, tail, total_L, 0, 0, vpr, tpb);
+      const int64_t e = r1 - r0 < g.cap ? r1 : r0 + g.cap;
+      int64_t row;
+      const int64_t copy = place(p, r0, r1, r0, e, row);
+      emit_rows<VEC, ADD, DT, MUL>(dense, x, out, r0, e, copy, row, vpr, 1 << lg, blockIdx.y,
+                                   gridDim.y);
     }
+    return;
+  }
+  const int64_t w = (blockIdx.x - g.list_blocks) * gridDim.y + blockIdx.y;
+  if (w >= g.windows) return;
+  const int64_t a = w * g.window, b = a + g.window < total_L ? a + g.window : total_L;
+  const int64_t head = clamp(off_at<I>(m, last, 0), 0);
+  const int64_t tail = clamp(off_at<I>(m, last, nlists), head);
+  // The list that row a lies in: only it can reach past its cap here, as one that
+  // starts later in the window has its first cap rows in it and beyond.
+  int64_t p = 0, r0 = 0, past = b, r1 = 0;
+  if (g.cap < total_L && a >= head && a < tail) {
+    p = wave_owner<I>(m, last, nlists, a);
+    r0 = clamp(off_at<I>(m, last, p), 0);
+    r1 = clamp(off_at<I>(m, last, p + 1), r0);
+    past = a > r0 + g.cap ? a : r0 + g.cap;
+    r1 = r1 < b ? r1 : b;
+  }
+  if (a >= head && b <= tail && past >= r1) return;  // the usual end
+#pragma unroll 1
+  for (int i = 0; i < 3; ++i) {  // rows before the first list, past the last, past a cap
+    const int64_t s = i == 0 ? a : (i == 2 ? past : (a > tail ? a : tail));
+    const int64_t e = i == 0 ? (b < head ? b : head) : (i == 1 ? b : r1);
+    int64_t copy = 0, row = 0;
+    if (s >= e) continue;
+    if (i == 2) copy = place(p, r0, clamp(off_at<I>(m, last, p + 1), r0), s, e, row);
+    emit_rows<VEC, ADD, DT, MUL>(dense, x, out, s, e, copy, row, vpr, 256, 0, 1);
   }
 }
 
 // ---- host side ------------------------------------------------------------
 
-// Threads per bag (2^lg) and grid: the smallest group that holds a full bag's
-// chunks in one round, kJagItems per thread, up to a block; bags in x, parts of
-// a bag in y (the kernels loop over what the grid leaves).
+// Threads per bag (2^lg) and grid: the smallest group that holds a usual bag's
+// chunks in one round, kJagItems per thread, up to a block; or one chunk per
+// thread, while all bags' threads are on the chip at once (a small call waits for
+// its slowest thread).  Bags in x, parts of a large bag in y (the kernels loop
+// over what the grid leaves).
 struct BagGrid {
   dim3 grid;
   int32_t lg;
 };
 
-BagGrid bag_grid(int64_t bags, int64_t chunks_per_bag) {
-  const int64_t chunks = chunks_per_bag > 0 ? chunks_per_bag : 1;
+BagGrid bag_grid(int64_t bags, int64_t usual_chunks, int64_t large_chunks) {
+  const int64_t resident = static_cast<int64_t>(num_cus()) * 2048;
   BagGrid g;
-  g.lg = chunks <= 16 * kJagItems ? 4 : (chunks <= 64 * kJagItems ? 6 : 8);
-  int64_t parts = ceil_div(chunks, static_cast<int64_t>(kJagItems) << g.lg);
-  if (parts > 64) parts = 64;
+  g.lg = 4;
+  while (g.lg < 8 && (usual_chunks > (int64_t(kJagItems) << g.lg) ||
+                      (usual_chunks > (int64_t(1) << g.lg) && bags << (g.lg + 2) <= resident)))
+    g.lg += 2;
+  int64_t parts = ceil_div(large_chunks, static_cast<int64_t>(kJagItems) << g.lg);
+  parts = parts < 1 ? 1 : (parts > 64 ? 64 : parts);
   int64_t x = ceil_div(bags, int64_t(1) << (8 - g.lg));
   if (x > (int64_t(1) << 30)) x = int64_t(1) << 30;
   g.grid = dim3(static_cast<uint32_t>(x), static_cast<uint32_t>(parts));
+  return g;
+}
+
+// Jagged outputs: groups by the mean list, parts by max_length within one and two
+// means (lists that max_length truncates are cleared whole; a padded dense far
+// longer than its lists would launch mostly blocks without rows).  A group takes
+// a list of up to eight times that (so that the windows of an ordinary batch, few
+// then, find nothing), or an even share of 1024 windows, or any list where all of
+// them together are 32 rounds of a group at most.  (2,560 lists of 5 rows of 64
+// columns under a max_length of 1000, copied back: 62 us with groups and parts by
+// max_length, 5.5; of 25 rows under 50, added in bf16: 17.0 and 10.5.)
+BagGrid list_grid(int64_t nlists, int64_t max_L, int64_t total_L, int64_t vpr, ListGrid& lg) {
+  const int64_t mean = ceil_div(total_L, nlists > 0 ? nlists : 1);
+  int64_t rows = max_L < mean ? mean : (max_L < 2 * mean ? max_L : 2 * mean);
+  if (rows * vpr < 16 * kJagItems) rows = ceil_div(16 * kJagItems, vpr);
+  BagGrid g = bag_grid(nlists, mean * vpr, rows * vpr);
+  const int64_t share = ceil_div(total_L, 1024);
+  const int64_t block_rows = ceil_div(8 * 256 * kJagItems, vpr);
+  lg.list_blocks = g.grid.x;
+  lg.cap = 8 * rows > share ? 8 * rows : share;
+  if (total_L * vpr <= (int64_t(32 * kJagItems) << g.lg)) lg.cap = total_L;
+  lg.window = share > block_rows ? share : block_rows;
+  if (lg.window > lg.cap) lg.window = lg.cap;
+  lg.windows = ceil_div(total_L, lg.window);
+  g.grid.x += static_cast<uint32_t>(ceil_div(lg.windows, static_cast<int64_t>(g.grid.y)));
   return g;
 }
 
@@ -412,7 +523,7 @@ extern "C" int mx_jagged_to_padded_dense(const void* values, int64_t elem_bytes,
   auto* o = static_cast<uint8_t*>(out);
   const int64_t max_L = max_lengths[num_jagged_dim - 1];
   const int64_t nbags = rows / max_L;  // rows > 0: max_L > 0
-  const BagGrid g = bag_grid(nbags, max_L * vpr);
+  const BagGrid g = bag_grid(nbags, max_L * vpr, max_L * vpr);
   const bool one = num_jagged_dim == 1 && g.lg == 8;
   MX_VEC_SWITCH(vec, {
     Chunk<V> pad;
@@ -455,7 +566,8 @@ static int jagged_output_op(const void* dense, int64_t elem_bytes, int64_t inner
   auto* o = static_cast<uint8_t*>(out);
   const int last = num_jagged_dim - 1;
   const int64_t nlists = offsets_numel[last] - 1;
-  const BagGrid g = bag_grid(nlists + 1, max_lengths[last] * vpr);
+  ListGrid lists;
+  const BagGrid g = list_grid(nlists, max_lengths[last], total_L, vpr, lists);
   const bool one = num_jagged_dim == 1 && g.lg == 8;
   if (x_values == nullptr) {
     MX_VEC_SWITCH(vec, {
@@ -464,7 +576,7 @@ static int jagged_output_op(const void* dense, int64_t elem_bytes, int64_t inner
                                                    : jagged_out_kernel<V, int32_t, false, F, false, true>)
                               : (offset_bytes == 8 ? jagged_out_kernel<V, int64_t, false, F, false, false>
                                                    : jagged_out_kernel<V, int32_t, false, F, false, false>);
-      kernel<<<g.grid, 256, 0, s>>>(d, nullptr, o, m, nlists, g.lg, total_L, vpr);
+      kernel<<<g.grid, 256, 0, s>>>(d, nullptr, o, m, nlists, g.lg, total_L, vpr, lists);
     });
     MX_LAUNCH_CHECK();
     return MX_OK;
@@ -480,7 +592,7 @@ static int jagged_output_op(const void* dense, int64_t elem_bytes, int64_t inner
                                    : jagged_out_kernel<V, int32_t, true, DTC, MULC, true>)      \
               : (offset_bytes == 8 ? jagged_out_kernel<V, int64_t, true, DTC, MULC, false>      \
                                    : jagged_out_kernel<V, int32_t, true, DTC, MULC, false>);    \
-      kernel<<<g.grid, 256, 0, s>>>(d, x, o, m, nlists, g.lg, total_L, vpr);                    \
+      kernel<<<g.grid, 256, 0, s>>>(d, x, o, m, nlists, g.lg, total_L, vpr, lists);                    \
     }                                                                                           \
   })
 #define MX_ADD_LAUNCH(DTC)    \
