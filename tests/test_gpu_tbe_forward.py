@@ -11,7 +11,7 @@ import torch
 
 import oracle as orc
 from mx_fbgemm import bench_inputs
-from tbe_helpers import random_tbe, tbe_forward_gpu, weight_offsets
+from tbe_helpers import gpu_us, random_tbe, tbe_forward_gpu, weight_offsets
 
 pytestmark = pytest.mark.gpu
 
@@ -273,3 +273,40 @@ def test_table_past_4gib(dev, wdtype, D):
         _exact(got, exp)
     del W, rows_used
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("wide,narrow", [(256, 32), (512, 64)])
+@pytest.mark.parametrize("weighted", [False, True])
+def test_wide_table_beside_narrow_ones(dev, wide, narrow, weighted):
+    """A table that holds nearly all of a small batch's lookups is read as fast
+    beside five narrow tables as alone (at most 1.7 times: their bags are the
+    batch's launch and a little; lanes and registers chosen for the narrow ones
+    took 1.8 to 2.8 times)."""
+    print(f"[case] tbe fwd {wide} beside {narrow} weighted={weighted}", flush=True)
+    rng = np.random.default_rng(wide)
+    B, E = 64, 20000
+    off1 = bench_inputs.offsets_from_lengths(rng.integers(50, 151, B))
+    narrow_len = rng.integers(0, 3, 5 * B)
+    off6 = np.concatenate([off1, off1[-1] + np.cumsum(narrow_len)]).astype(np.int64)
+    idx = rng.integers(0, E, int(off6[-1]))
+    both = bench_inputs.TbeInput(T=6, E=[E] * 6, D=[wide] + [narrow] * 5, B=B, indices=idx,
+                                 offsets=off6)
+    alone = bench_inputs.TbeInput(T=1, E=[E], D=[wide], B=B, indices=idx[: off1[-1]], offsets=off1)
+
+    def us(inp):
+        W = torch.randn(sum(e * d for e, d in zip(inp.E, inp.D)), device=dev)
+        args = (torch.from_numpy(weight_offsets(inp)).to(dev),
+                torch.from_numpy(inp.D_offsets).to(dev), inp.total_D, wide,
+                torch.from_numpy(inp.indices).to(dev), torch.from_numpy(inp.offsets).to(dev), 0)
+        empty, pl = torch.zeros(0, device=dev), torch.zeros(inp.T, dtype=torch.int32, device=dev)
+        tail = (torch.zeros(0, dtype=torch.int32, device=dev), empty, 0, False)
+        if weighted:
+            iw = torch.rand(inp.N, device=dev)
+            return gpu_us(lambda: torch.ops.fbgemm.split_embedding_codegen_forward_weighted_cuda(
+                W, empty, empty, pl, *args, iw, *tail))
+        return gpu_us(lambda: torch.ops.fbgemm.split_embedding_codegen_forward_unweighted_cuda(
+            W, empty, empty, pl, *args, *tail))
+
+    t6, t1 = us(both), us(alone)
+    print(f"beside {t6:.1f} us, alone {t1:.1f}", flush=True)
+    assert t6 <= 1.7 * t1

@@ -280,9 +280,7 @@ constexpr int fwd_rows() {
 // (c*G + k)*4 .. +4 (float4 loads: a D=128 row is one 512 B access of 32
 // lanes).  Several bags per wave keep several independent offsets -> indices
 // -> rows chains in flight; each column is still summed in index order.
-// MIXED: tables of different widths; G fits the narrow ones and a wave takes
-// 1, 2 or NCH chunks per lane by its bags' own widths.
-template <typename I, typename WT, int G, int NCH, bool MIXED, bool WEIGHTED, bool OUT_F16>
+template <typename I, typename WT, int G, int NCH, bool WEIGHTED, bool OUT_F16>
 __global__ void __launch_bounds__(256)
     __attribute__((amdgpu_waves_per_eu(fwd_waves<I, NCH, WEIGHTED>())))
     tbe_fwd_group_kernel(const WT* __restrict__ W, const int64_t* __restrict__ w_off,
@@ -351,21 +349,8 @@ __global__ void __launch_bounds__(256)
   const bool one_table = __all(t == tw);  // wave-uniform
   const __amdgpu_buffer_rsrc_t rsrc = table_rsrc(W + w_off[tw]);
 
-  const int64_t obase = bm.out_base(bag, b, D0);
-#define MX_POOL(N)                                                                              \
-  pool_bag<I, WT, G, N, fwd_rows<N>(), WEIGHTED, OUT_F16>(Wt, rsrc, one_table, D, indices, iw, \
-                                                          start, end, pooling, out, obase, g, k)
-  if constexpr (MIXED) {
-    if (__all(D <= 4 * G))  // wave-uniform
-      MX_POOL(1);
-    else if (__all(D <= 8 * G))
-      MX_POOL(2);
-    else
-      MX_POOL(NCH);
-  } else {
-    MX_POOL(NCH);
-  }
-#undef MX_POOL
+  pool_bag<I, WT, G, NCH, fwd_rows<NCH>(), WEIGHTED, OUT_F16>(
+      Wt, rsrc, one_table, D, indices, iw, start, end, pooling, out, bm.out_base(bag, b, D0), g, k);
 }
 
 // Gradient of the per-sample weights of a weighted lookup:
@@ -513,51 +498,48 @@ __global__ void __launch_bounds__(256)
 #undef MX_DOT
 }
 
-// Tables of different widths (a fixed batch says so: total_D) whose mean is at
-// most five eighths of the widest: there the lanes that fit the widest rows
-// are half idle or more (six widths from 32 to 256: 22.6 -> 20.9 us).  Nearer the
-// widest, more lanes per bag keep more rows in flight (128 and 64 in turn: a
-// training step 137.0 us, 138.5 mixed).
+// For the per-sample-weight gradient: tables of different widths (a fixed batch
+// says so: total_D) whose mean is at most five eighths of the widest.  There the
+// lanes that fit the widest rows are half idle or more: 24 tables of six widths
+// up to 256, 4096 bags each, 92.9 us with them and 53.2 by each wave's widths,
+// 1024 bags 26.1 and 15.9.  A few dozen bags, or a wide table with nearly all of
+// the lookups, rather want its many lanes (6 tables, 256 and 5 x 32 columns, 64
+// bags: 38.5 us, 60.7 here, 64.8 by a reduction per row as before).  The forward
+// has no such instances: they took its waves from eight per SIMD to four and a
+// wide table's bags from four waves to one (the 64 bags: 17.0 us, 47.5 with them;
+// the 24 tables 57.8 and 51.5).
 bool mixed_widths(const BagMap& bm, int32_t T, int32_t max_D) {
   return bm.total_D > 0 && max_D > 64 && 8 * bm.total_D <= 5ll * T * max_D;
 }
 
-template <typename I, typename WT, int G, int NCH, bool MIXED, bool WEIGHTED, bool OUT_F16>
+template <typename I, typename WT, int G, int NCH, bool WEIGHTED, bool OUT_F16>
 void launch_fwd_group(hipStream_t s, const WT* W, const int64_t* w_off, const int32_t* D_off,
                       const BagMap& bm, const void* idx, const void* off, int32_t pooling,
                       const float* iw, void* out, int64_t nbags) {
   constexpr int P = 64 / G;
   const int64_t grid = ceil_div(nbags, kWavesPerBlock * P);
-  tbe_fwd_group_kernel<I, WT, G, NCH, MIXED, WEIGHTED, OUT_F16>
+  tbe_fwd_group_kernel<I, WT, G, NCH, WEIGHTED, OUT_F16>
       <<<dim3(static_cast<uint32_t>(grid)), 256, 0, s>>>(
           W, w_off, D_off, bm, static_cast<const I*>(idx), static_cast<const I*>(off), pooling, iw,
           out, nbags);
 }
 
 template <typename I, typename WT, bool WEIGHTED, bool OUT_F16>
-int dispatch_fwd(hipStream_t s, int32_t T, int32_t max_D, const WT* W, const int64_t* w_off,
+int dispatch_fwd(hipStream_t s, int32_t max_D, const WT* W, const int64_t* w_off,
                  const int32_t* D_off, const BagMap& bm, const void* idx, const void* off,
                  int32_t pooling, const float* iw, void* out, int64_t nbags) {
-#define MX_FWD_G(G, NCH, MIXED) \
-  launch_fwd_group<I, WT, G, NCH, MIXED, WEIGHTED, OUT_F16>(s, W, w_off, D_off, bm, idx, off, \
-                                                            pooling, iw, out, nbags)
-  const bool mixed = mixed_widths(bm, T, max_D);
+#define MX_FWD_G(G, NCH) \
+  launch_fwd_group<I, WT, G, NCH, WEIGHTED, OUT_F16>(s, W, w_off, D_off, bm, idx, off, pooling, iw, out, nbags)
   if (max_D <= 64)
-    MX_FWD_G(16, 1, false);  // 4 bags per wave
-  else if (mixed && max_D <= 256)
-    MX_FWD_G(16, 4, true);
-  else if (mixed && max_D <= 512)
-    MX_FWD_G(32, 4, true);
+    MX_FWD_G(16, 1);  // 4 bags per wave
   else if (max_D <= 128)
-    MX_FWD_G(32, 1, false);  // 2 bags per wave, one D=128 row per 32 lanes x 16 B
+    MX_FWD_G(32, 1);  // 2 bags per wave, one D=128 row per 32 lanes x 16 B
   else if (max_D <= 256)
-    MX_FWD_G(64, 1, false);
+    MX_FWD_G(64, 1);
   else if (max_D <= 512)
-    MX_FWD_G(64, 2, false);
-  else if (mixed)
-    MX_FWD_G(64, 4, true);
+    MX_FWD_G(64, 2);
   else
-    MX_FWD_G(64, 4, false);
+    MX_FWD_G(64, 4);
 #undef MX_FWD_G
   return MX_OK;
 }
@@ -714,7 +696,7 @@ int tbe_forward_impl(const void* weights, int32_t weights_ty, const int64_t* wei
   auto* s = as_stream(stream);
   const bool w = indice_weights != nullptr;
   const bool h = out_dtype == MX_SPARSE_FP16;
-#define MX_ARGS(WT) s, T, max_D, static_cast<const WT*>(weights), weights_offsets, D_offsets, bm, \
+#define MX_ARGS(WT) s, max_D, static_cast<const WT*>(weights), weights_offsets, D_offsets, bm, \
                 indices, offsets, pooling_mode, indice_weights, out, nbags
 #define MX_FWD_W(I, WT)                                                                          \
   if (w)                                                                                         \
