@@ -63,6 +63,21 @@ def test_row_codec_lane_edges(dev, bits, rows, D):
     (words per lane, lanes per row, the wide kernel), partial last words, and
     row counts that leave groups idle; encode and decode bit-exact."""
     print(f"[case] row codec bits={bits} rows={rows} D={D}", flush=True)
+    _check_row_codec(dev, bits, rows, D)
+
+
+@pytest.mark.parametrize("bits", [2, 4, 8, "fused8"])
+@pytest.mark.parametrize("rows,D", [(65407, 9), (65537, 31), (32767, 62), (32769, 65),
+                                    (16385, 129), (8191, 255), (8193, 257), (4097, 513)])
+def test_row_codec_rows_per_group(dev, bits, rows, D):
+    """Row counts either side of two blocks per CU, where a group takes several
+    rows instead of one, at widths that leave partial words, with a last group
+    of fewer rows; encode and decode bit-exact."""
+    print(f"[case] row codec groups bits={bits} rows={rows} D={D}", flush=True)
+    _check_row_codec(dev, bits, rows, D)
+
+
+def _check_row_codec(dev, bits, rows, D):
     x = _rows(np.random.default_rng(D), rows, D)
     ops = torch.ops.fbgemm
     for src in (torch.from_numpy(x), torch.from_numpy(x).half()):
