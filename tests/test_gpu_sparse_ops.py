@@ -168,12 +168,15 @@ def test_permute_2d_sparse_data_sizes(dev, T, B, Tp, ldtype):
 
 @pytest.mark.parametrize("T,Tp,B,maxlen", [(1, 1, 1, 40), (40, 40, 100, 30), (1024, 1024, 3, 5),
                                            (1025, 1024, 3, 5), (300, 1025, 2, 5), (5, 7, 8192, 4),
-                                           (5, 7, 8193, 4), (2, 3, 40000, 3)])
+                                           (5, 7, 8193, 4), (2, 3, 40000, 3), (1024, 1024, 16, 5),
+                                           (1025, 1024, 16, 5), (512, 512, 15, 5), (513, 512, 15, 5),
+                                           (3, 3, 16, 7), (3, 4, 60, 100), (10, 10, 600, 100)])
 @pytest.mark.parametrize("idtype", [torch.int32, torch.int64])
 def test_permute_2d_by_feature(dev, T, Tp, B, maxlen, idtype):
     """Either side of the feature counts and bag parts at which the per-feature
-    sums take over from the cumsums, blocks inside one feature and over many
-    short ones, and a given output size below the lengths' sum."""
+    sums take over from the cumsums, blocks of one index per thread and of more,
+    inside one feature, over two or three and over many short ones, and a given
+    output size below the lengths' sum."""
     print(f"[case] permute_2D by feature T={T} Tp={Tp} B={B} i={idtype}", flush=True)
     rng = np.random.default_rng(T * 31 + B)
     lengths = rng.integers(0, maxlen, (T, B))
