@@ -86,6 +86,21 @@ def test_workspace_sizes_grow(lib):
     assert 0 < g(1000, 23) < a
 
 
+@pytest.mark.parametrize("N", [1, 16, 17, 32, 33, 66, 1000, 99_991, 10_000_000])
+def test_backward_workspace_partials(lib, N):
+    """The backward's room for chunk partials, in rows of max_D floats: enough for
+    the worst batch (runs of the length with the most 32-occurrence chunks each),
+    and no more than 2/33 per position and one, whatever the widths."""
+    f = lib.mx_tbe_backward_workspace_bytes
+    f.restype = ctypes.c_size_t
+    f.argtypes = [ctypes.c_int64, ctypes.c_int32, ctypes.c_int32]
+    rows = (f(N, 23, 128) - f(N, 23, 64)) // (64 * 4)  # multiples of 256 bytes each
+    worst = max((N // n) * -(-n // 32) + (-(-(N % n) // 32) if N % n > 16 else 0)
+                for n in range(17, min(N, 400) + 1)) if N > 16 else 0
+    assert worst <= rows <= 2 * N // 33 + 1
+    assert rows <= N // 32 + N // 25 + 2  # chunks from 25 occurrences on
+
+
 def test_bad_arguments_rejected_before_any_launch(lib):
     lib.mx_last_error.restype = ctypes.c_char_p
     P = ctypes.c_void_p

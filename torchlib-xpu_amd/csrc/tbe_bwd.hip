@@ -98,9 +98,12 @@ int32_t long_run(int32_t T, int32_t max_D, int64_t total_D) {
 constexpr int kChunk = 32;                            // occurrences per chunk
 // One-pass scans per backward: run heads, chunk layout.
 constexpr int kScanSlots = 2;
-// Upper bound of the chunk count: sum over runs longer than kLongMin of
-// ceil(len / kChunk) <= N / kChunk + (number of such runs).
-int64_t max_chunks(int64_t N) { return N / kChunk + N / (kLongMin + 1) + 2; }
+// Upper bound of the chunk count (and one, so that it is not 0): the sum of
+// ceil(len / kChunk) over the runs longer than kLongMin.  A run of len
+// occurrences has at most 2/33 chunks per occurrence: 1/17 for 17 .. 32 of them,
+// 2/33 for 33, and m/(32m - 31) at most, which falls, for m > 2 chunks.
+int64_t max_chunks(int64_t N) { return 2 * N / 33 + 1; }
+static_assert(kLongMin >= 16 && kChunk == 32, "the chunk bound");
 
 __device__ __forceinline__ uint32_t digit_mask(int bits, int p) {
   const int nb = bits - p * kRadixBits;
