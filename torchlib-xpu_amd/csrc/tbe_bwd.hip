@@ -83,12 +83,14 @@ constexpr int64_t kSegRow = static_cast<int64_t>(kHistCopies) * kMaxPasses * kRa
 constexpr int64_t kLinTile = 256 * kLinItems;         // positions per linearize block
 // Runs longer than long_run() are chunked.  A wave's four short runs last as
 // long as the longest (two occurrences per round): 24 instead of 32 moves the
-// 13-16-round runs to the chunk path (config 3: 161.1 -> 158.8 us; 12, 16 and
-// 20 were within 1 us of it, 8 slower).  Where the update's rows cost more per
-// occurrence -- wide ones, or widths the lanes do not divide -- 16 is better
-// (96-column sequences 150.5 -> 146.6 us, tables of 256, 200 and 168 columns
-// 201.6 -> 197.4, 256 123.4 -> 121.5), at full width up to 128 columns 24 stays
-// (64 columns: 152.6, 156.5 with 16; config 3: 201.3, 202.5).
+// 13-16-round runs to the chunk path (config 3: 161.1 -> 158.8 us; 8 slower).
+// The line between 16 and 24 is worth 1 % where it shows at all: the full-width
+// instances of up to 128 columns (launch_width; 64 and 128 columns in every
+// table of a fixed or a sequence batch), the cheapest per occurrence, are better
+// with 24 (config 3: 201.7 us, 203.7 with 16), instances whose lanes test their
+// columns with 16 (96-column sequences 136.2, 138.3 with 24; weighted tables of
+// six widths 168.3, 170.1).  No difference either way: 8, 16, 32, 60, 124, 256,
+// 512 and 1024 columns, and variable batches of 64 and 128 (360.1 and 359.1).
 constexpr int kLongNarrow = 24;
 constexpr int kLongMin = 16;
 int32_t long_run(int32_t T, int32_t max_D, int64_t total_D) {
@@ -914,7 +916,10 @@ struct ChunkEpi {
 // kSmallMax: eight keys per lane, the most that leave the ranks in registers
 // and the keys in 64 KB of LDS.
 constexpr int kSmallMax = 8192;
-constexpr int64_t kSmallMaxBags = 65536;  // each thread reads this / 1024 offset pairs at most
+// kSmallMaxBags: each thread reads this / 1024 offset pairs at most.  A training
+// step of 8000 positions, the chain of launches and one block: 4096 bags 53.8 and
+// 37.8 us, 16384 56.5 and 53.0, 65536 66.5 and 67.6 (of 500 positions 59.1, 34.5).
+constexpr int64_t kSmallMaxBags = 65536;
 
 struct SmallSort {
   const int64_t* hsc;
