@@ -70,14 +70,17 @@ def test_transpose_keys_outside_their_table_sort_globally(dev):
     _check_transpose(dev, inp, torch.int32)
 
 
-def test_transpose_too_few_key_bits(dev):
+@pytest.mark.parametrize("B", [300, 500])
+def test_transpose_too_few_key_bits(dev, B):
     """With total_hash_size_bits below the keys' width the sort orders keys by
     their low bits (as a radix sort over those bits does, across features):
     per-feature segments would not, so the sort runs over the whole batch and
-    matches the oracle's masked stable sort."""
-    print("[case] transpose, 11 key bits for 3,000 rows", flush=True)
+    matches the oracle's masked stable sort; in one block (up to 8192 positions)
+    and in the chain of launches."""
+    print(f"[case] transpose, 11 key bits for 3,000 rows, B={B}", flush=True)
     rng = np.random.default_rng(11)
-    inp = random_tbe(rng, 3, 300, [4] * 3, [1000, 1000, 1000], 20)
+    inp = random_tbe(rng, 3, B, [4] * 3, [1000, 1000, 1000], 20)
+    assert (inp.N > 8192) == (B == 500), inp.N
     bits = 11  # 2^11 = 2048 < 3000 rows
     nb = orc.info_B_num_bits(inp.T, inp.B)
     exp = orc.transpose_embedding_input(inp.hash_size_cumsum, inp.B, nb, bits, inp.indices,
@@ -430,18 +433,21 @@ def _shared_tables(rng, ftm, rows, dims, B, max_L, dup=False):
 @pytest.mark.parametrize("weighted", [False, True])
 @pytest.mark.parametrize("dup", [False, True])
 @pytest.mark.parametrize("ftm", [[0, 1, 0, 2, 1], [0, 0, 1, 1, 2]])
-def test_backward_shared_tables(dev, pooling, weighted, dup, ftm):
+@pytest.mark.parametrize("B", [120, 200])
+def test_backward_shared_tables(dev, pooling, weighted, dup, ftm, B):
     """Features sharing tables (fbgemm's feature_table_map; hash_size_cumsum
     then decreases, and the sort runs over the whole batch, or repeats, and
-    each table's features sort as one segment): one run per row of a shared
+    each table's features sort as one segment; up to 8192 positions one block
+    sorts either): one run per row of a shared
     table, each occurrence summing its own feature's
     gradient columns (MEAN: its own bag length); duplicate-heavy batches reach
     the chunked long-run path.  Transpose bit-exact, update within rtol 1e-5."""
-    print(f"[case] shared tables ftm={ftm} pool={pooling} weighted={weighted} dup={dup}",
+    print(f"[case] shared tables ftm={ftm} pool={pooling} weighted={weighted} dup={dup} B={B}",
           flush=True)
     rng = np.random.default_rng(50 + pooling + 2 * weighted + 4 * dup + 8 * ftm[1])
     rows, dims = [300, 200, 50], [64, 32, 128]
-    inp, w_off, hsc, m1_off, bits = _shared_tables(rng, ftm, rows, dims, 120, 30, dup)
+    inp, w_off, hsc, m1_off, bits = _shared_tables(rng, ftm, rows, dims, B, 30, dup)
+    assert (inp.N > 8192) == (B == 200), inp.N
     nb = orc.info_B_num_bits(inp.T, inp.B)
     exp = orc.transpose_embedding_input(hsc, inp.B, nb, bits, inp.indices, inp.offsets)
     got = torch.ops.fbgemm.transpose_embedding_input(
@@ -482,12 +488,13 @@ def test_backward_shared_tables(dev, pooling, weighted, dup, ftm):
 
 
 @pytest.mark.parametrize("weighted", [False, True])
-def test_module_training_step_shared_tables(dev, weighted):
+@pytest.mark.parametrize("B", [24, 700])
+def test_module_training_step_shared_tables(dev, weighted, B):
     """SplitTableBatchedEmbeddingBagsCodegen(specs, feature_table_map=[0, 1, 0]):
     forward bit-exact against the oracle on the per-feature arrays, and one
     fused update per row of the shared table (vs the oracle pinned to torch
     autograd on shared tables)."""
-    print(f"[case] module shared tables weighted={weighted}", flush=True)
+    print(f"[case] module shared tables weighted={weighted} B={B}", flush=True)
     from mx_fbgemm import ComputeDevice, EmbeddingLocation, PoolingMode
     from mx_fbgemm.split_table_batched_embeddings_ops_training import (
         SplitTableBatchedEmbeddingBagsCodegen,
@@ -499,7 +506,8 @@ def test_module_training_step_shared_tables(dev, weighted):
                                                 learning_rate=0.05, eps=1e-6, device=dev,
                                                 weights_init=(-0.5, 0.5))
     rng = np.random.default_rng(61 + weighted)
-    inp, w_off, hsc, m1_off, bits = _shared_tables(rng, ftm, rows, dims, 24, 12, dup=True)
+    inp, w_off, hsc, m1_off, bits = _shared_tables(rng, ftm, rows, dims, B, 12, dup=True)
+    assert (inp.N > 8192) == (B == 700), inp.N
     assert tbe.weights_offsets.tolist() == w_off.tolist()
     assert tbe.hash_size_cumsum.tolist() == hsc.tolist()
     W0 = tbe.weights_dev.detach().cpu().numpy().copy()
@@ -1011,11 +1019,13 @@ def test_counter_region_matches_workspace_counters(dev):
     (the graph-capture form), and both match the oracle."""
     rng = np.random.default_rng(77)
     cases = [
-        random_tbe(rng, 40, 24, [16] * 40, [300] * 40, 12),
-        random_tbe(rng, 3, 200, [4, 64, 256], [50, 2000, 40], 30),
-        random_tbe(rng, 1, 300, [128], [7], 40, dup_heavy=True),
+        random_tbe(rng, 40, 60, [16] * 40, [300] * 40, 12),
+        random_tbe(rng, 3, 300, [4, 64, 256], [50, 2000, 40], 30),
+        random_tbe(rng, 1, 700, [128], [7], 40, dup_heavy=True),
         random_tbe(rng, 5, 700, [4] * 5, [2 ** 20, 3, 100, 9, 2 ** 21], 10),
     ]
+    # One block sorts fewer positions, without counters.
+    assert min(inp.N for inp in cases) > 8192, [inp.N for inp in cases]
     for i, inp in enumerate(cases):
         print(f"[case] counter region, batch {i} (T={inp.T})", flush=True)
         got_region, _ = _backward_case(dev, inp, i % 2, seed=i)

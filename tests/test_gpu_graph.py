@@ -255,13 +255,17 @@ def test_fp16_stochastic_rounding_graph_replays_draw_fresh_bits(dev):
             f"replay {k} rounded with other bits than the eager step"
 
 
-def test_nobag_training_step_graph_replays_match_eager(dev):
-    """PoolingMode NONE: the nobag forward, the nobag backward and an nbit nobag lookup, captured
-    together; every replay equals the eager step bit for bit."""
-    print("[case] graph-captured nobag forward + backward + nbit nobag, 4 replays", flush=True)
+@pytest.mark.parametrize("B", [128, 500])
+def test_nobag_training_step_graph_replays_match_eager(dev, B):
+    """PoolingMode NONE: the nobag forward, the nobag backward (its sort in one block and in the
+    chain of launches) and an nbit nobag lookup, captured together; every replay equals the eager
+    step bit for bit."""
+    print(f"[case] graph-captured nobag forward + backward + nbit nobag, 4 replays, B={B}",
+          flush=True)
     rng = np.random.default_rng(6)
     D = 64
-    inp = random_tbe(rng, 3, 128, [D] * 3, [400, 3, 900], 20)
+    inp = random_tbe(rng, 3, B, [D] * 3, [400, 3, 900], 20)
+    assert (inp.N > 8192) == (B == 500), inp.N
     nW = sum(E * D for E in inp.E)
     W0 = torch.from_numpy(rng.uniform(-0.5, 0.5, nW).astype(np.float32)).to(dev)
     grads = [torch.from_numpy(rng.normal(0, 1e-2, (inp.N, D)).astype(np.float32)).to(dev)

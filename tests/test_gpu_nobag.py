@@ -344,20 +344,23 @@ def test_inference_module_nobag(dev, out):
     np.testing.assert_array_equal(g, exp.view(np.uint32) if kind == 0 else exp.view(np.uint16))
 
 
-@pytest.mark.parametrize("layout", ["empty_first", "empty_middle", "empty_last", "shared_table"])
+@pytest.mark.parametrize("layout", ["empty_first", "empty_middle", "empty_last", "shared_table",
+                                    "shared_decreasing"])
 def test_nobag_sort_segments(dev, layout):
     """A sequence batch sorts in per-feature segments: whole features without
     positions (first, middle, last) and two features sharing one table (equal
     hash_size_cumsum entries: one segment), each feature over several
-    3072-key sort tiles; backward and transpose against the oracle."""
+    3072-key sort tiles; a table shared by features 0 and 2 (hash_size_cumsum
+    decreases) makes the sort global.  Backward and transpose against the oracle."""
     print(f"[case] nobag sort segments {layout}", flush=True)
-    seed = {"empty_first": 1, "empty_middle": 2, "empty_last": 3, "shared_table": 4}[layout]
+    seed = {"empty_first": 1, "empty_middle": 2, "empty_last": 3, "shared_table": 4,
+            "shared_decreasing": 5}[layout]
     rng = np.random.default_rng(700 + seed)
     T, B, D = 4, 1500, 64
-    rows = [300, 400, 400, 60]
+    rows = [300, 400, 300 if layout == "shared_decreasing" else 400, 60]
     lengths = rng.integers(0, 11, size=(T, B))
     lengths[rng.random((T, B)) < 0.2] = 0
-    if layout != "shared_table":
+    if layout.startswith("empty"):
         lengths[{"empty_first": 0, "empty_middle": 2, "empty_last": 3}[layout]] = 0
     offsets = bench_inputs.offsets_from_lengths(lengths.reshape(-1))
     indices = np.concatenate([rng.integers(0, rows[t], int(lengths[t].sum())) for t in range(T)])
@@ -365,6 +368,11 @@ def test_nobag_sort_segments(dev, layout):
         hsc = np.array([0, 300, 300, 700, 760], np.int64)
         w_off = np.array([0, 300 * D, 300 * D, 700 * D], np.int64)
         m1_off = np.array([0, 300, 300, 700], np.int64)
+        n_rows = 760
+    elif layout == "shared_decreasing":
+        hsc = np.array([0, 300, 0, 700, 760], np.int64)
+        w_off = np.array([0, 300 * D, 0, 700 * D], np.int64)
+        m1_off = np.array([0, 300, 0, 700], np.int64)
         n_rows = 760
     else:
         hsc = bench_inputs.offsets_from_lengths(np.asarray(rows, np.int64))
@@ -409,14 +417,15 @@ def test_nobag_sort_segments(dev, layout):
 
 @pytest.mark.parametrize("N", [3000, 12000])
 @pytest.mark.parametrize("layout", ["head", "tail", "all", "overlap"])
-def test_nobag_positions_outside_bags(dev, N, layout):
+@pytest.mark.parametrize("index_dtype", [torch.int64, torch.int32])
+def test_nobag_positions_outside_bags(dev, N, layout, index_dtype):
     """Positions before the first bag count as table 0's and positions past the
     last as the last table's, each with its own gradient row (all: no bag holds
     any position, every offset is N), either side of 8192 positions.  In
     `overlap` table 1 (the rows of table 0, one sort segment) ends before it
     starts: the segments do not hold the positions of their tables, so the
     batch sorts as one."""
-    print(f"[case] nobag outside bags N={N} {layout}", flush=True)
+    print(f"[case] nobag outside bags N={N} {layout} {index_dtype}", flush=True)
     rng = np.random.default_rng(N)
     T, B, D = 3, 4, 36
     hsc = np.array([0, 0, 50, 120], np.int64)
@@ -436,7 +445,7 @@ def test_nobag_positions_outside_bags(dev, N, layout):
     empty = torch.zeros(0, device=dev)
     pl = torch.zeros(T, dtype=torch.int32, device=dev)
     hsc_d = torch.from_numpy(hsc).to(dev)
-    idx_d, off_d = torch.from_numpy(indices).to(dev), torch.from_numpy(offsets).to(dev)
+    idx_d, off_d = (torch.from_numpy(a).to(dev, index_dtype) for a in (indices, offsets))
     out = torch.ops.fbgemm.transpose_embedding_input(hsc_d, bits, idx_d, off_d, True)
     exp = orc.transpose_embedding_input_nobag(hsc, B, bits, indices, covering)
     assert int(out[5].item()) == exp["num_runs"]
