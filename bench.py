@@ -377,7 +377,7 @@ def wl_jagged(args, dev) -> Workload:
         unit="GB/s", steps=[step], units=[alg / 1e9], alg_bytes=[alg], dtype="fp32",
         config={"workload": "config1: jagged round trip, B=512 D=128 max_L=64, len~U{0..64}",
                 "B": B, "D": D, "max_L": L, "total_L": total},
-        kernel="j2pd1_kernel + jagged_out1_kernel (one round trip)", profile="jagged_config1",
+        kernel="j2pd_kernel + jagged_out_kernel (one round trip)", profile="jagged_config1",
         cpu=cpu, cold_steps=cold)
 
 
@@ -605,7 +605,7 @@ def wl_permute(args, dev) -> Workload:
         units=[N], alg_bytes=[compulsory], dtype="int64",
         config={"workload": "config2 batch, permute_2D_sparse_data (features reversed, "
                             "int64 lengths and indices, no weights)", "T": T, "B": B, "N": N},
-        kernel="whole op (permuted lengths, two complete cumsums, the copy)",
+        kernel="whole op (feature sums and permuted lengths, the copy)",
         profile="permute_2d_config2", cpu=cpu, cold_steps=cold, roof_bytes=compulsory,
         roof_bytes_kind="compulsory bytes: indices and lengths each read and written once")
 
@@ -755,7 +755,7 @@ def wl_nobag_backward(args, dev) -> Workload:
         unit="lookups/s", steps=[step], units=[inp.N], alg_bytes=[alg], dtype="fp32",
         config={"workload": "config3 batch, PoolingMode NONE backward: grad_output [N, 128]",
                 "T": T, "E": E, "D": D, "B": B, "N": inp.N, "unique_rows": U},
-        kernel="whole nobag backward (layout + transpose + segment reduce + update)",
+        kernel="whole nobag backward (transpose + segment reduce + update)",
         profile="tbe_bwd_nobag_config3", cpu=cpu, cold_steps=cold)
 
 
