@@ -12,7 +12,7 @@
 //   * each repaired entry (offset or index) adds one to warning[0];
 //   * FATAL repairs nothing and only counts (the host raises on a non-zero
 //     count); NONE does nothing.
-// Work: one launch, or two from kOneTile bags on, and no zeroed state.  A tile
+// Work: one launch, or two above kOneTile bags, and no zeroed state.  A tile
 // kernel takes, one wave per tile, the maximum of the clamped offsets of every
 // tile of `tile` bags (a smaller batch is one tile, which needs none).  Then a
 // block owns `bpb` consecutive bags (32 to 256, so that the grid fills the
